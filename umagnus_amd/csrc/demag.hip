@@ -23,6 +23,8 @@
 #include <type_traits>
 
 #include "batch.hpp"
+#include "demag_reg.hpp"
+#include "demag_x4.hpp"
 #include "fft_ct.hpp"
 #include "field.hpp"
 #include "sim.hpp"
@@ -59,25 +61,6 @@ __device__ __forceinline__ void run_fft(C2<T> *lds, const C2<T> *twl, int nl, co
 // ---------------------------------------------------------------------------
 // X forward: rows of real data -> half spectrum (packed two-for-one R2C).
 // ---------------------------------------------------------------------------
-template <typename T>
-struct XArgs {
-  FftLen f;               // complex length n = Px/2
-  const C2<T> *tw2;       // exp(-2 pi i k / Px), k in [0, Px)
-  int mode;               // 0: mu0*Ms*vol*m rows of Nx valid reals; 1: raw real rows of Px
-  int nl;                 // lines per work-group
-  FastDiv fhalf;          // n/2 + 1
-  int Nx;                 // valid reals per input row
-  int rows;               // input rows per component
-  FastDiv fRy;            // input rows per z-plane (Ny, or Py for mode 1)
-  int Py;                 // spectrum rows per z-plane
-  int Hp;                 // spectrum row pitch
-  long in_pitch;          // input row pitch (reals)
-  const T *src[3];
-  Par<T> Ms;
-  const T *vol;
-  C2<T> *out[3];
-};
-
 template <typename T, int CN, int CNL>
 struct BXfwd {
   using Args = XArgs<T>;
@@ -170,16 +153,6 @@ __global__ __launch_bounds__(FFT_NT) void k_xfwd(XArgs<T> a) { BXfwd<T, CN, CNL>
 // ---------------------------------------------------------------------------
 // X inverse: half spectrum rows -> real rows (C2R), keeping x < Nx.
 // ---------------------------------------------------------------------------
-template <typename T>
-struct XiArgs {
-  FftLen f;
-  const C2<T> *tw2;
-  int nl, Nx, rows, Py, Hp;
-  FastDiv fhalf, fRy;
-  const C2<T> *in[3];
-  T *dst[3];
-};
-
 template <typename T, int CN, int CNL>
 struct BXinv {
   using Args = XiArgs<T>;
@@ -352,51 +325,6 @@ __global__ __launch_bounds__(FFT_NT) void k_xinv_odd(XiArgs<T> a) { BXinvOdd<T>:
 // the stride-(A+1) reads are bank-conflict free.
 // ---------------------------------------------------------------------------
 constexpr int XF4_NT = 128;
-
-// Twiddle table of the step between the two register transforms of a
-// four-step pass: W_n^(r k2) (r < R, k2 < K) at [r][k2], rows padded by one
-// entry.  Loading and storing are split so that a kernel issues the table's
-// global loads after its data loads and writes the table once both arrived:
-// no memory round trip of its own ahead of the data.
-template <typename T, int R, int K, int NT>
-struct TwStage {
-  static constexpr int Q = (R * K + NT - 1) / NT;
-  C2<T> v[Q];
-  __device__ __forceinline__ void load(const C2<T> *tw, int step) {   // tw[step r k2] = W_n^(r k2)
-  #pragma unroll
-    for (int q = 0; q < Q; q++) {
-      const int i = (int)threadIdx.x + q * NT;
-      if ((R * K) % NT == 0 || i < R * K) {
-        const int r = i / K, k2 = i - r * K;
-        v[q] = tw[step * r * k2];
-      }
-    }
-  }
-  __device__ __forceinline__ void store(C2<T> *lds) const {
-  #pragma unroll
-    for (int q = 0; q < Q; q++) {
-      const int i = (int)threadIdx.x + q * NT;
-      if ((R * K) % NT == 0 || i < R * K) {
-        const int r = i / K, k2 = i - r * K;
-        lds[r * (K + 1) + k2] = v[q];
-      }
-    }
-  }
-};
-
-// exp(dir * 2 pi i j / n); constant once the caller's loops are unrolled
-template <typename T>
-__device__ __forceinline__ C2<T> cexpi(int j, int n, int dir) {
-  const double ang = 2.0 * M_PI * (double)j / (double)n;
-  return C2<T>{T(__builtin_cos(ang)), T(dir * __builtin_sin(ang))};
-}
-
-template <int N> struct X4Shape;
-template <> struct X4Shape<64> { static constexpr int A = 8, B = 8; };
-template <> struct X4Shape<128> { static constexpr int A = 8, B = 16; };
-template <> struct X4Shape<256> { static constexpr int A = 16, B = 16; };
-template <> struct X4Shape<512> { static constexpr int A = 16, B = 32; };
-template <> struct X4Shape<1024> { static constexpr int A = 32, B = 32; };
 
 // inverse: half spectrum X[k], k = 0..n -> real rows, x < Nx = n:
 // Z'[k] = (X[k] + conj X[n-k]) + i W_2n^-k (X[k] - conj X[n-k]), z = IDFT_n(Z'),
@@ -602,30 +530,24 @@ struct ColArgs {
   C2<T> *buf[3];
 };
 
-template <typename T, int DIR, int CN, int CNL>
+template <typename T, int DIR>
 struct BColfft {
   using Args = ColArgs<T>;
   static constexpr int NT = FFT_NT, MINB = 1;
   static __device__ __forceinline__ void run(const ColArgs<T> &a, uint3 blockIdx, uint3 gridDim) {
-    constexpr int EPT = FftEpt<T>::value;
+    constexpr int SL = FftEpt<T>::value;
     extern __shared__ __align__(16) unsigned char smem_[];
     C2<T> *lds = (C2<T> *)smem_;
-    const int n = CN > 0 ? CN : a.f.n, nl = CN > 0 ? CNL : a.nl, total = nl * n;
-    C2<T> *twl = lds + nl * n;
-    if constexpr (CN > 0) {
-      const C2<T> *tw = (const C2<T> *)a.f.tw;
-      for (int g = threadIdx.x; g < CN; g += FFT_NT) twl[g] = tw[g];
-    }
+    const int n = a.f.n, nl = a.nl, total = nl * n;
     const int kx0 = blockIdx.x * nl;
     C2<T> *base = a.buf[blockIdx.z] + (long)blockIdx.y * a.pstride;
-    constexpr int SL = CN > 0 ? (CN * CNL + FFT_NT - 1) / FFT_NT : EPT;
     C2<T> v[SL];
   #pragma unroll
     for (int s = 0; s < SL; s++) {
       const int g = threadIdx.x + s * FFT_NT;
       v[s] = C2<T>{T(0), T(0)};
       if (g < total) {
-        const int e = cdiv<CNL>(g, a.fnl), l = g - e * nl;
+        const int e = (int)a.fnl.div(g), l = g - e * nl;
         const int kx = kx0 + l;
         if (kx < a.H && e < a.nvalid) v[s] = base[(long)e * a.estride + kx];
       }
@@ -636,20 +558,20 @@ struct BColfft {
       if (g < total) lds[g] = v[s];   // element-major: g = e*nl + l
     }
     __syncthreads();
-    run_fft<T, CN, CNL, DIR, 1, 1>(lds, twl, nl, a.fnl, a.f);
+    lds_fft<T, DIR, 1>(lds, nl, a.fnl, 1, nl, a.f);
   #pragma unroll
     for (int s = 0; s < SL; s++) {
       const int g = threadIdx.x + s * FFT_NT;
       if (g < total) {
-        const int e = cdiv<CNL>(g, a.fnl), l = g - e * nl;
+        const int e = (int)a.fnl.div(g), l = g - e * nl;
         const int kx = kx0 + l;
         if (kx < a.H && e < a.nout) base[(long)e * a.estride + kx] = lds[g];
       }
     }
   }
 };
-template <typename T, int DIR, int CN, int CNL>
-__global__ __launch_bounds__(FFT_NT) void k_colfft(ColArgs<T> a) { BColfft<T, DIR, CN, CNL>::run(a, hw_bid(), hw_grid()); }
+template <typename T, int DIR>
+__global__ __launch_bounds__(FFT_NT) void k_colfft(ColArgs<T> a) { BColfft<T, DIR>::run(a, hw_bid(), hw_grid()); }
 
 // ---------------------------------------------------------------------------
 // Register four-step column pass for P = A*A (A in 8, 16, 32): C adjacent kx
@@ -671,14 +593,6 @@ __global__ __launch_bounds__(FFT_NT) void k_colfft(ColArgs<T> a) { BColfft<T, DI
 #ifndef UM_COLY_ZB
 #define UM_COLY_ZB 1
 #endif
-
-// Work-group index permuted so that the tiles one XCD runs (linear ids w,
-// w+8, w+16, ... are dispatched to the same XCD) are adjacent in memory and
-// share their 128-byte lines in that XCD's L2.
-__device__ __forceinline__ int xcd_tile(int w, int total) {
-  const int q = total >> 3, full = q << 3;
-  return w >= full ? w : (w & 7) * q + (w >> 3);
-}
 
 template <typename T, int A, int DIR, int C, bool HALF, int ZB>
 struct BColy {
@@ -1524,14 +1438,14 @@ struct TwTable {
       pp *= r[i];
     }
   }
-  void make(int n, hipStream_t s) {
+  void make(int n, UnitRoots &roots, hipStream_t s) {
     len.n = n;
     len.fn.init(n > 0 ? n : 1);
     schedule(0);
     std::vector<C2<T>> h(n > 0 ? n : 1);
-    for (int m = 0; m < n; m++) {
-      const long double ang = -2.0L * 3.14159265358979323846264338327950288L * (long double)m / (long double)n;
-      h[m] = C2<T>{(T)cosl(ang), (T)sinl(ang)};
+    if (n > 0) {
+      const auto &w = roots.get(n);
+      for (int m = 0; m < n; m++) h[m] = C2<T>{(T)w[m].x, (T)w[m].y};
     }
     buf.alloc(sizeof(C2<T>) * h.size());
     UM_HIP(hipMemcpyAsync(buf.p, h.data(), sizeof(C2<T>) * h.size(), hipMemcpyHostToDevice, s));
@@ -1541,34 +1455,26 @@ struct TwTable {
 };
 
 // ---- launch dispatch: compile-time instantiations for the hot sizes ------------
-// Lines per work-group of each specialised length (LDS budget ~40-72 KiB so two
-// or more work-groups share a CU); other lengths use the generic kernels.
+// Lines (columns) per work-group of the compiled lengths: X rows of 32, 48, 96
+// and 192 points and the convolution of narrow films (fewer than CONV2_H
+// columns) in FP32, whose few work-groups wait on the address and twiddle
+// chains that a compile-time length shortens (96 x 96: 13 us a convolution
+// against 14 with register-stage X rows, 17 with both passes), and the 64-point
+// convolution in FP64 (512 x 512 x 32: 1.48 ms against 1.76).  The other
+// lengths run the register-stage passes, or the generic engine where a length
+// has no split.
+constexpr int CONV2_H = 384;
 template <typename T> struct CtTable;
-// The 32/48/96/192-point X, 96/192/384-point Y and Pz = 3/5/7 Z entries serve
-// small grids with Nx, Ny in {32, 48, 96, 192} and Nz <= 4 (ensembles).
 template <> struct CtTable<float> {
-  static int x(int n) {
-    switch (n) { case 32: return 32; case 48: return 32; case 64: return 32; case 96: return 16; case 128: return 16;
-                 case 192: return 16; case 256: return 16; case 512: return 8; case 1024: return 4; }
-    return 0;
-  }
-  static int col(int n) {
-    switch (n) { case 64: return 32; case 96: return 16; case 128: return 16; case 192: return 8; case 256: return 16;
-                 case 384: return 8; case 512: return 8; case 1024: return 8; case 2048: return 4; }
-    return 0;
-  }
-  static int conv3(int n) { switch (n) { case 3: return 32; case 5: return 32; case 7: return 32; case 16: return 16; case 32: return 16; case 64: return 16; } return 0; }
-  static int conv2(int n) {
-    switch (n) { case 64: return 16; case 96: return 16; case 128: return 16; case 192: return 8; case 256: return 8;
-                 case 384: return 4; case 512: return 4; }
-    return 0;
+  static int x(int n) { switch (n) { case 32: return 32; case 48: return 32; case 96: return 16; case 192: return 16; } return 0; }
+  static int conv(int n, bool is2d, int H) {
+    const bool len = n == 64 || n == 96 || n == 128 || n == 192 || n == 256 || n == 384 || n == 512;
+    return is2d && len && H < CONV2_H ? 1 : 0;
   }
 };
 template <> struct CtTable<double> {
-  static int x(int n) { switch (n) { case 256: return 8; case 512: return 4; } return 0; }
-  static int col(int n) { switch (n) { case 512: return 4; case 1024: return 4; } return 0; }
-  static int conv3(int n) { switch (n) { case 16: return 8; case 64: return 8; } return 0; }
-  static int conv2(int n) { switch (n) { case 256: return 4; case 512: return 2; } return 0; }
+  static int x(int) { return 0; }
+  static int conv(int n, bool is2d, int) { return !is2d && n == 64 ? 8 : 0; }
 };
 
 template <typename B> struct BTag { using type = B; };
@@ -1633,22 +1539,6 @@ template <typename T>
 static void launch_xfwd(const XArgs<T> &a, int n, int nl, dim3 grid, hipStream_t s) {
   const size_t ct = sizeof(C2<T>) * ((size_t)nl * n + 2 * n);
   if constexpr (std::is_same<T, float>::value) {
-    UM_CT_CASE((BXfwd<float, 64, 32>), (k_xfwd<float, 64, 32>), 64, 32, ct)
-    UM_CT_CASE((BXfwd<float, 128, 16>), (k_xfwd<float, 128, 16>), 128, 16, ct)
-    UM_CT_CASE((BXfwd<float, 256, 16>), (k_xfwd<float, 256, 16>), 256, 16, ct)
-    UM_CT_CASE((BXfwd<float, 512, 8>), (k_xfwd<float, 512, 8>), 512, 8, ct)
-    UM_CT_CASE((BXfwd<float, 1024, 4>), (k_xfwd<float, 1024, 4>), 1024, 4, ct)
-    // few rows (small grids): fewer rows per work-group, more work-groups
-    UM_CT_CASE((BXfwd<float, 64, 8>), (k_xfwd<float, 64, 8>), 64, 8, ct)
-    UM_CT_CASE((BXfwd<float, 64, 1>), (k_xfwd<float, 64, 1>), 64, 1, ct)
-    UM_CT_CASE((BXfwd<float, 128, 4>), (k_xfwd<float, 128, 4>), 128, 4, ct)
-    UM_CT_CASE((BXfwd<float, 128, 1>), (k_xfwd<float, 128, 1>), 128, 1, ct)
-    UM_CT_CASE((BXfwd<float, 256, 4>), (k_xfwd<float, 256, 4>), 256, 4, ct)
-    UM_CT_CASE((BXfwd<float, 256, 1>), (k_xfwd<float, 256, 1>), 256, 1, ct)
-    UM_CT_CASE((BXfwd<float, 512, 2>), (k_xfwd<float, 512, 2>), 512, 2, ct)
-    UM_CT_CASE((BXfwd<float, 512, 1>), (k_xfwd<float, 512, 1>), 512, 1, ct)
-    UM_CT_CASE((BXfwd<float, 1024, 1>), (k_xfwd<float, 1024, 1>), 1024, 1, ct)
-    // small grids of the other X lengths
     UM_CT_CASE((BXfwd<float, 32, 32>), (k_xfwd<float, 32, 32>), 32, 32, ct)
     UM_CT_CASE((BXfwd<float, 32, 8>), (k_xfwd<float, 32, 8>), 32, 8, ct)
     UM_CT_CASE((BXfwd<float, 32, 1>), (k_xfwd<float, 32, 1>), 32, 1, ct)
@@ -1661,9 +1551,6 @@ static void launch_xfwd(const XArgs<T> &a, int n, int nl, dim3 grid, hipStream_t
     UM_CT_CASE((BXfwd<float, 192, 16>), (k_xfwd<float, 192, 16>), 192, 16, ct)
     UM_CT_CASE((BXfwd<float, 192, 4>), (k_xfwd<float, 192, 4>), 192, 4, ct)
     UM_CT_CASE((BXfwd<float, 192, 1>), (k_xfwd<float, 192, 1>), 192, 1, ct)
-  } else {
-    UM_CT_CASE((BXfwd<double, 256, 8>), (k_xfwd<double, 256, 8>), 256, 8, ct)
-    UM_CT_CASE((BXfwd<double, 512, 4>), (k_xfwd<double, 512, 4>), 512, 4, ct)
   }
   launch_b<BXfwd<T, 0, 0>>(k_xfwd<T, 0, 0>, grid, dim3(FFT_NT), sizeof(C2<T>) * nl * n, s, a);
   UM_HIP(hipGetLastError());
@@ -1673,11 +1560,6 @@ static void launch_xinv(const XiArgs<T> &a, int n, int nl, dim3 grid, hipStream_
   if (four_step && launch_xi4<T>(a, n, s)) return;
   const size_t ct = sizeof(C2<T>) * ((size_t)nl * n + 2 * n);
   if constexpr (std::is_same<T, float>::value) {
-    UM_CT_CASE((BXinv<float, 64, 32>), (k_xinv<float, 64, 32>), 64, 32, ct)
-    UM_CT_CASE((BXinv<float, 128, 16>), (k_xinv<float, 128, 16>), 128, 16, ct)
-    UM_CT_CASE((BXinv<float, 256, 16>), (k_xinv<float, 256, 16>), 256, 16, ct)
-    UM_CT_CASE((BXinv<float, 512, 8>), (k_xinv<float, 512, 8>), 512, 8, ct)
-    UM_CT_CASE((BXinv<float, 1024, 4>), (k_xinv<float, 1024, 4>), 1024, 4, ct)
     UM_CT_CASE((BXinv<float, 32, 32>), (k_xinv<float, 32, 32>), 32, 32, ct)
     UM_CT_CASE((BXinv<float, 32, 8>), (k_xinv<float, 32, 8>), 32, 8, ct)
     UM_CT_CASE((BXinv<float, 32, 1>), (k_xinv<float, 32, 1>), 32, 1, ct)
@@ -1690,33 +1572,17 @@ static void launch_xinv(const XiArgs<T> &a, int n, int nl, dim3 grid, hipStream_
     UM_CT_CASE((BXinv<float, 192, 16>), (k_xinv<float, 192, 16>), 192, 16, ct)
     UM_CT_CASE((BXinv<float, 192, 4>), (k_xinv<float, 192, 4>), 192, 4, ct)
     UM_CT_CASE((BXinv<float, 192, 1>), (k_xinv<float, 192, 1>), 192, 1, ct)
-  } else {
-    UM_CT_CASE((BXinv<double, 256, 8>), (k_xinv<double, 256, 8>), 256, 8, ct)
-    UM_CT_CASE((BXinv<double, 512, 4>), (k_xinv<double, 512, 4>), 512, 4, ct)
   }
   launch_b<BXinv<T, 0, 0>>(k_xinv<T, 0, 0>, grid, dim3(FFT_NT), sizeof(C2<T>) * nl * n, s, a);
   UM_HIP(hipGetLastError());
 }
 template <typename T, int DIR>
 static void launch_col(const ColArgs<T> &a, int n, int nl, dim3 grid, hipStream_t s) {
-  const size_t ct = sizeof(C2<T>) * ((size_t)nl * n + n);
-  if constexpr (std::is_same<T, float>::value) {
-    UM_CT_CASE((BColfft<float, DIR, 64, 32>), (k_colfft<float, DIR, 64, 32>), 64, 32, ct)
-    UM_CT_CASE((BColfft<float, DIR, 128, 16>), (k_colfft<float, DIR, 128, 16>), 128, 16, ct)
-    UM_CT_CASE((BColfft<float, DIR, 256, 16>), (k_colfft<float, DIR, 256, 16>), 256, 16, ct)
-    UM_CT_CASE((BColfft<float, DIR, 512, 8>), (k_colfft<float, DIR, 512, 8>), 512, 8, ct)
-    UM_CT_CASE((BColfft<float, DIR, 1024, 8>), (k_colfft<float, DIR, 1024, 8>), 1024, 8, ct)
-    UM_CT_CASE((BColfft<float, DIR, 2048, 4>), (k_colfft<float, DIR, 2048, 4>), 2048, 4, ct)
-    UM_CT_CASE((BColfft<float, DIR, 96, 16>), (k_colfft<float, DIR, 96, 16>), 96, 16, ct)
-    UM_CT_CASE((BColfft<float, DIR, 192, 8>), (k_colfft<float, DIR, 192, 8>), 192, 8, ct)
-    UM_CT_CASE((BColfft<float, DIR, 384, 8>), (k_colfft<float, DIR, 384, 8>), 384, 8, ct)
-  } else {
-    UM_CT_CASE((BColfft<double, DIR, 512, 4>), (k_colfft<double, DIR, 512, 4>), 512, 4, ct)
-    UM_CT_CASE((BColfft<double, DIR, 1024, 4>), (k_colfft<double, DIR, 1024, 4>), 1024, 4, ct)
-  }
-  launch_b<BColfft<T, DIR, 0, 0>>(k_colfft<T, DIR, 0, 0>, grid, dim3(FFT_NT), sizeof(C2<T>) * nl * n, s, a);
+  launch_b<BColfft<T, DIR>>(k_colfft<T, DIR>, grid, dim3(FFT_NT), sizeof(C2<T>) * nl * n, s, a);
   UM_HIP(hipGetLastError());
 }
+template <typename T>
+static bool coly_len(int P) { return P == 64 || P == 256 || (P == 1024 && sizeof(T) == 4); }
 // Register four-step Y pass when P = A*A (A = 8, 16, 32 in FP32; 8, 16 in FP64)
 // and the column is either half zero-padded or full; false: use launch_col.
 template <typename T, int DIR>
@@ -1764,240 +1630,23 @@ template <typename T>
 static void launch_conv(const ConvArgs<T> &a, int n, int B, dim3 grid, hipStream_t s) {
   const int nl = B;  // UM_CT_CASE compares (n, nl)
   const size_t ct = sizeof(C2<T>) * ((size_t)3 * B * n + n);
-  if (!a.is2d) {
-    if constexpr (std::is_same<T, float>::value) {
-      UM_CT_CASE((BConv<float, 16, 16>), (k_conv<float, 16, 16>), 16, 16, ct)
-      UM_CT_CASE((BConv<float, 32, 16>), (k_conv<float, 32, 16>), 32, 16, ct)
-      UM_CT_CASE((BConv<float, 64, 16>), (k_conv<float, 64, 16>), 64, 16, ct)
-      UM_CT_CASE((BConv<float, 3, 32>), (k_conv<float, 3, 32>), 3, 32, ct)     // Pz = 2 Nz - 1 for Nz = 2, 3, 4
-      UM_CT_CASE((BConv<float, 5, 32>), (k_conv<float, 5, 32>), 5, 32, ct)
-      UM_CT_CASE((BConv<float, 7, 32>), (k_conv<float, 7, 32>), 7, 32, ct)
-    } else {
-      UM_CT_CASE((BConv<double, 16, 8>), (k_conv<double, 16, 8>), 16, 8, ct)
-      UM_CT_CASE((BConv<double, 64, 8>), (k_conv<double, 64, 8>), 64, 8, ct)
+  if constexpr (std::is_same<T, float>::value) {
+    if (a.is2d) {
+      UM_CT_CASE((BConv<float, 64, 1>), (k_conv<float, 64, 1>), 64, 1, ct)
+      UM_CT_CASE((BConv<float, 96, 1>), (k_conv<float, 96, 1>), 96, 1, ct)
+      UM_CT_CASE((BConv<float, 128, 1>), (k_conv<float, 128, 1>), 128, 1, ct)
+      UM_CT_CASE((BConv<float, 192, 1>), (k_conv<float, 192, 1>), 192, 1, ct)
+      UM_CT_CASE((BConv<float, 256, 1>), (k_conv<float, 256, 1>), 256, 1, ct)
+      UM_CT_CASE((BConv<float, 384, 1>), (k_conv<float, 384, 1>), 384, 1, ct)
+      UM_CT_CASE((BConv<float, 512, 1>), (k_conv<float, 512, 1>), 512, 1, ct)
     }
   } else {
-    if constexpr (std::is_same<T, float>::value) {
-      UM_CT_CASE((BConv<float, 64, 16>), (k_conv<float, 64, 16>), 64, 16, ct)
-      UM_CT_CASE((BConv<float, 128, 16>), (k_conv<float, 128, 16>), 128, 16, ct)
-      UM_CT_CASE((BConv<float, 256, 8>), (k_conv<float, 256, 8>), 256, 8, ct)
-      UM_CT_CASE((BConv<float, 512, 4>), (k_conv<float, 512, 4>), 512, 4, ct)
-      // narrow spectra (small grids): fewer columns per work-group
-      UM_CT_CASE((BConv<float, 64, 4>), (k_conv<float, 64, 4>), 64, 4, ct)
-      UM_CT_CASE((BConv<float, 64, 1>), (k_conv<float, 64, 1>), 64, 1, ct)
-      UM_CT_CASE((BConv<float, 128, 4>), (k_conv<float, 128, 4>), 128, 4, ct)
-      UM_CT_CASE((BConv<float, 128, 1>), (k_conv<float, 128, 1>), 128, 1, ct)
-      UM_CT_CASE((BConv<float, 256, 2>), (k_conv<float, 256, 2>), 256, 2, ct)
-      UM_CT_CASE((BConv<float, 256, 1>), (k_conv<float, 256, 1>), 256, 1, ct)
-      UM_CT_CASE((BConv<float, 512, 1>), (k_conv<float, 512, 1>), 512, 1, ct)
-      UM_CT_CASE((BConv<float, 96, 16>), (k_conv<float, 96, 16>), 96, 16, ct)
-      UM_CT_CASE((BConv<float, 96, 4>), (k_conv<float, 96, 4>), 96, 4, ct)
-      UM_CT_CASE((BConv<float, 96, 1>), (k_conv<float, 96, 1>), 96, 1, ct)
-      UM_CT_CASE((BConv<float, 192, 8>), (k_conv<float, 192, 8>), 192, 8, ct)
-      UM_CT_CASE((BConv<float, 192, 2>), (k_conv<float, 192, 2>), 192, 2, ct)
-      UM_CT_CASE((BConv<float, 192, 1>), (k_conv<float, 192, 1>), 192, 1, ct)
-      UM_CT_CASE((BConv<float, 384, 4>), (k_conv<float, 384, 4>), 384, 4, ct)
-      UM_CT_CASE((BConv<float, 384, 1>), (k_conv<float, 384, 1>), 384, 1, ct)
-    } else {
-      UM_CT_CASE((BConv<double, 256, 4>), (k_conv<double, 256, 4>), 256, 4, ct)
-      UM_CT_CASE((BConv<double, 512, 2>), (k_conv<double, 512, 2>), 512, 2, ct)
-    }
+    if (!a.is2d) UM_CT_CASE((BConv<double, 64, 8>), (k_conv<double, 64, 8>), 64, 8, ct)
   }
   launch_b<BConv<T, 0, 0>>(k_conv<T, 0, 0>, grid, dim3(FFT_NT), sizeof(C2<T>) * 3 * B * n, s, a);
   UM_HIP(hipGetLastError());
 }
 #undef UM_CT_CASE
-
-// ---------------------------------------------------------------------------
-// X inverse fused with the four-cell effective field + torque (FP32).  A
-// work-group of XF_NT threads inverts R rows (y0 .. y0+R-1 of one z plane) of
-// all three components with the register four-step of k_xi4 (3R lines, G per
-// 32-lane group), leaves the real B_demag lines in LDS, then evaluates the
-// effective field and torque of those R x Nx cells: B_demag never touches HBM.
-// Work-groups run z fastest (tile w -> y block w / Nz, plane w % Nz), so the
-// z +- 1 rows of m that the stencil reads were just read by the neighbouring
-// work-groups of the same XCD and are still in its L2.
-// ---------------------------------------------------------------------------
-constexpr int XF_NT = 192;
-
-template <int N> struct XFShape {
-  static constexpr int A = X4Shape<N>::A, B = X4Shape<N>::B, G = B / A;
-  static constexpr int R = 64 * G / B;    // rows per work-group
-  static constexpr int L = 3 * R;         // lines (component-major: line = c R + j)
-  static_assert(L / G * B == XF_NT, "the lines of R rows fill the work-group");
-};
-
-template <typename T>
-struct XiFieldArgs {
-  XiArgs<T> x;
-  FieldArgs<T> f;
-};
-// TH = false (no thermal term, checked on the host) at N = 512: at most 128
-// VGPRs without spills (the launch bound's second argument is the minimum
-// number of waves per SIMD with hipcc), so five work-groups share a CU
-// instead of four; the other lengths would spill under that bound
-template <typename T, int N, bool REG, int EX, bool UNI, bool TH>
-struct BXi4Field {
-  using Args = XiFieldArgs<T>;
-  static constexpr int NT = XF_NT, MINB = (!TH && N == 512) ? 4 : 1;
-  static __device__ __forceinline__ void run(const XiFieldArgs<T> &a, uint3 blockIdx, uint3 gridDim) {
-    const XiArgs<T> &x = a.x;
-    const FieldArgs<T> &f = a.f;
-    using S = XFShape<N>;
-    constexpr int A = S::A, B = S::B, G = S::G, R = S::R, TS = B * (A + 1), HB = B / 2;
-    static_assert(S::L * N <= S::L * TS, "B_demag lines fit the transpose space");
-    // the transpose moves the real, then the imaginary parts (half the LDS of
-    // complex entries: more work-groups per CU); afterwards line (c, j) holds
-    // B_demag_c of row j, x < N
-    __shared__ __align__(16) T ldr[S::L * TS];
-    // twiddles of the step between the two transforms, W_N^(n1 k2) at
-    // [n1][k2] (rows padded by one entry: the A rows fall on distinct banks);
-    // read from LDS instead of global memory, their latency stays out of the
-    // transform
-    __shared__ C2<T> twb[A * (B + 1)];
-    for (int i = threadIdx.x; i < A * B; i += XF_NT) {
-      const int r = i / B, k2 = i - r * B;
-      twb[r * (B + 1) + k2] = x.tw2[2 * r * k2];
-    }
-    const int Ny = (int)x.fRy.d, Nz = x.rows / Ny;
-    const int w = xcd_tile(blockIdx.x, gridDim.x);
-    const int yb = w / Nz, z = w - yb * Nz, y0 = yb * R;
-    const int grp = threadIdx.x / B, l = threadIdx.x % B;
-    C2<T> v[B];
-    const int h1 = l / A, n1 = l % A, line1 = grp * G + h1;
-    {
-      const int c = line1 / R, y = y0 + (line1 - c * R);
-  #pragma unroll
-      for (int n2 = 0; n2 < B; n2++) v[n2] = C2<T>{T(0), T(0)};
-      if (y < Ny) {
-        // component base selected from the uniform arguments (an indexed read
-        // of x.in would be a per-lane load ahead of every spectrum load)
-        const C2<T> *inc = c == 0 ? x.in[0] : c == 1 ? x.in[1] : x.in[2];
-        const C2<T> *irow = inc + ((long)z * x.Py + y) * x.Hp;
-        // two halves of loads: half the staging registers live at a time
-  #pragma unroll
-        for (int hb = 0; hb < 2; hb++) {
-          C2<T> xk[HB], xn[HB];
-  #pragma unroll
-          for (int q = 0; q < HB; q++) {
-            const int k = n1 + A * (hb * HB + q);
-            xk[q] = irow[k];
-            xn[q] = irow[N - k];
-          }
-  #pragma unroll
-          for (int q = 0; q < HB; q++) {
-            const int n2 = hb * HB + q, k = n1 + A * n2;
-            const C2<T> sm = cadd(xk[q], cconj(xn[q])), d = csub(xk[q], cconj(xn[q]));
-            const C2<T> t = cmul(cconj(x.tw2[k]), d);
-            v[n2] = C2<T>{sm.x - t.y, sm.y + t.x};
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      dft<B, +1>(v);
-      __syncthreads();   // the twiddle table is complete
-  #pragma unroll
-      for (int k2 = 1; k2 < B; k2++) v[k2] = cmul(v[k2], cconj(twb[n1 * (B + 1) + k2]));   // W_n^-(n1 k2)
-    }
-    C2<T> u[G][A];
-    T *tw = ldr + line1 * TS + n1;
-  #pragma unroll
-    for (int k2 = 0; k2 < B; k2++) tw[k2 * (A + 1)] = v[k2].x;
-    __syncthreads();
-  #pragma unroll
-    for (int h = 0; h < G; h++) {
-      const T *t = ldr + (grp * G + h) * TS + l * (A + 1);
-  #pragma unroll
-      for (int q = 0; q < A; q++) u[h][q].x = t[q];
-    }
-    __syncthreads();
-  #pragma unroll
-    for (int k2 = 0; k2 < B; k2++) tw[k2 * (A + 1)] = v[k2].y;
-    __syncthreads();
-  #pragma unroll
-    for (int h = 0; h < G; h++) {
-      const T *t = ldr + (grp * G + h) * TS + l * (A + 1);
-  #pragma unroll
-      for (int q = 0; q < A; q++) u[h][q].y = t[q];
-    }
-    T *bl = ldr;
-    __syncthreads();   // every transpose read is done: the space now takes the real lines
-  #pragma unroll
-    for (int h = 0; h < G; h++) {
-      dft<A, +1>(u[h]);
-      T *o = bl + (grp * G + h) * N;
-  #pragma unroll
-      for (int k1 = 0; k1 < A / 2; k1++) *(float2 *)(o + 2 * (l + B * k1)) = float2{u[h][k1].x, u[h][k1].y};
-    }
-    __syncthreads();
-    constexpr int NGX = N / 4, NG = R * NGX;
-    for (int g = threadIdx.x; g < NG; g += XF_NT) {
-      const int j = g / NGX, gx = g - j * NGX, y = y0 + j;
-      if (y >= Ny) continue;
-      T bdv[3][4];
-  #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const float4 b = *(const float4 *)(bl + (c * R + j) * N + 4 * gx);
-        bdv[c][0] = b.x; bdv[c][1] = b.y; bdv[c][2] = b.z; bdv[c][3] = b.w;
-      }
-      field_group4<T, REG, EX, false, UNI, false, TH>(f, 4 * gx, y, z, bdv);   // registers over instructions
-    }
-  }
-};
-template <typename T, int N, bool REG, int EX, bool UNI, bool TH>
-__global__ __launch_bounds__(XF_NT, (BXi4Field<T, N, REG, EX, UNI, TH>::MINB)) void k_xi4_field(XiFieldArgs<T> a) {
-  BXi4Field<T, N, REG, EX, UNI, TH>::run(a, hw_bid(), hw_grid());
-}
-
-// whether the fused kernel covers these field terms and buffers: the
-// four-cell kernel's terms without spin-transfer torques or bulk DMI, every
-// per-cell array aligned to four cells
-template <typename T>
-static bool xi4_field_ok(const FieldArgs<T> &a, int n) {
-  if (!std::is_same<T, float>::value || a.g.Nx != n || a.g.Nx % 4) return false;
-  if (n != 64 && n != 128 && n != 256 && n != 512 && n != 1024) return false;
-  if (a.exch_mode == 3 || a.has_zl || a.has_sl) return false;
-  auto al = [](const void *p) { return ((uintptr_t)p & (4 * sizeof(T) - 1)) == 0; };
-  for (int c = 0; c < 3; c++) {
-    if (!al(a.m[c])) return false;
-    if (a.tau[0] && !al(a.tau[c])) return false;
-    if (a.beff[0] && !al(a.beff[c])) return false;
-  }
-  return !a.regions || ((uintptr_t)a.regions & 3) == 0;
-}
-
-template <typename T>
-static void launch_xi4_field(const XiArgs<T> &a, const FieldArgs<T> &f, int n, hipStream_t s) {
-  if constexpr (std::is_same<T, float>::value) {
-    const int Ny = a.fRy.d, Nz = a.rows / Ny;
-    const bool reg = f.regions != nullptr, uni = field_uniform(f), th = f.has_therm != 0;
-    auto go = [&](auto tag, auto kern, int R) {
-      using K = typename decltype(tag)::type;
-      const dim3 grid((unsigned)(((Ny + R - 1) / R) * Nz));
-      launch_b<K>(kern, grid, dim3(XF_NT), 0, s, XiFieldArgs<T>{a, f});
-      UM_HIP(hipGetLastError());
-    };
-// the thermal-free variants only for uniform parameters (the hot case);
-// per-cell parameters without a thermal term take the TH = true kernel
-#define UM_XF2(CN, RG, E)                                                                                      \
-  { if (uni && !th) go(BTag<BXi4Field<T, CN, RG, E, true, false>>{}, k_xi4_field<T, CN, RG, E, true, false>,    \
-                       XFShape<CN>::R);                                                                          \
-    else if (uni) go(BTag<BXi4Field<T, CN, RG, E, true, true>>{}, k_xi4_field<T, CN, RG, E, true, true>,         \
-                     XFShape<CN>::R);                                                                            \
-    else go(BTag<BXi4Field<T, CN, RG, E, false, true>>{}, k_xi4_field<T, CN, RG, E, false, true>, XFShape<CN>::R); }
-#define UM_XF(CN)                                                                                    \
-  if (n == CN) {                                                                                     \
-    if (f.exch_mode == 0) { if (reg) UM_XF2(CN, true, 0) else UM_XF2(CN, false, 0) }                 \
-    else if (f.exch_mode == 1) { if (reg) UM_XF2(CN, true, 1) else UM_XF2(CN, false, 1) }            \
-    else { if (reg) UM_XF2(CN, true, 2) else UM_XF2(CN, false, 2) }                                  \
-    return;                                                                                          \
-  }
-    UM_XF(64) UM_XF(128) UM_XF(256) UM_XF(512) UM_XF(1024)
-#undef UM_XF
-#undef UM_XF2
-  }
-  throw Error(UM_EUNSUP, "fused X inverse: unsupported length");
-}
 
 static bool fused_field_default() {
   const char *e = std::getenv("UMHIP_FUSED_FIELD");
@@ -2079,6 +1728,11 @@ template <typename T>
 struct DemagPlan : DemagBase {
   int H, Hp, Hk, is2d, KHy, KHz;   // Hk: tensor row pitch (H rounded up to 128 bytes)
   TwTable<T> tx, ty, tz, tx2;   // tx: length Px/2, tx2: length Px (post-processing), ty, tz
+  // register-stage passes (demag_reg.hpp): X rows, Y columns, convolution axis
+  RegTab<T> rx, ry, rc;
+  DevBuf rtw;                   // their twiddle tables
+  UnitRoots roots;              // host side, while the plan is built
+  bool rshort = false;
   DevBuf spec[3];               // per component: Nz*Py*Hp complex
   DevBuf kern;                  // 6 x H*KHy*KHz of T
   // launch schedule (static tables, or the autotuner's choice): X forward and
@@ -2119,10 +1773,10 @@ struct DemagPlan : DemagBase {
     Hp = (H + al - 1) / al * al;
     KHy = P[1] / 2 + 1;
     KHz = P[2] / 2 + 1;
-    tx.make(P[0] / 2, s);
-    tx2.make(P[0], s);
-    ty.make(P[1], s);
-    tz.make(P[2], s);
+    tx2.make(P[0], roots, s);
+    tx.make(P[0] / 2, roots, s);
+    ty.make(P[1], roots, s);
+    tz.make(P[2], roots, s);
     nl_x = xodd ? lines_for(P[0]) : CtTable<T>::x(P[0] / 2);
     if (!nl_x) nl_x = lines_for(P[0] / 2);
     // small grids: trade rows per work-group for work-groups while the X pass
@@ -2136,19 +1790,12 @@ struct DemagPlan : DemagBase {
     }
     if (xodd || !CtTable<T>::x(P[0] / 2)) nl_x = spread(nl_x, (long)N[1] * N[2], 3);
     nl_xi = nl_x;
-    nl_y = CtTable<T>::col(P[1]);
     // the Y columns of a 3D grid run Nz planes deep: fuller groups pay there
-    if (!nl_y) nl_y = spread(std::min(lines_for(P[1]), 64), H, 3L * N[2], SMALL_GRID_WG / 6);
+    nl_y = spread(std::min(lines_for(P[1]), 64), H, 3L * N[2], SMALL_GRID_WG / 6);
 
     zreg = !is2d && P[2] == 2 * N[2] && ConvZTable<T>::has(N[2]);
     const int convlen = is2d ? P[1] : P[2];
-    B_conv = is2d ? CtTable<T>::conv2(convlen) : CtTable<T>::conv3(convlen);
-    if (is2d && B_conv && std::is_same<T, float>::value) {
-      for (int b : {B_conv / 4, 1}) {   // narrow spectra: more work-groups, as for the X pass
-        if (b < 1 || (H + B_conv - 1) / B_conv >= SMALL_GRID_WG) break;
-        B_conv = b;
-      }
-    }
+    B_conv = CtTable<T>::conv(convlen, is2d, H);
     if (!B_conv) {
       const int bmax = std::min(lines_for(convlen) / 3, 32);
       UM_REQUIRE(bmax >= 1, UM_EUNSUP, "convolution axis too long");
@@ -2158,6 +1805,7 @@ struct DemagPlan : DemagBase {
     }
     UM_REQUIRE(B_conv * (convlen / 2 + 1) <= FFT_NT * CONV_QK, UM_EUNSUP, "convolution prefetch slots exceeded");
     UM_REQUIRE(3 * B_conv * convlen <= FFT_NT * FftEpt<T>::value, UM_EUNSUP, "convolution tile exceeds LDS budget");
+    setup_reg(s);
     const size_t sc = is2d ? (size_t)N[1] * Hp : (size_t)N[2] * P[1] * Hp;
     for (int c = 0; c < 3; c++) spec[c].alloc(sizeof(C2<T>) * sc);
     Hk = (H + al2 - 1) / al2 * al2;
@@ -2165,15 +1813,35 @@ struct DemagPlan : DemagBase {
     kern.alloc(sizeof(T) * 6 * kcount);
   }
 
+  // register-stage passes (demag_reg.hpp) for the lengths without a compiled kernel
+  void setup_reg(hipStream_t s) {
+    // their byte offsets within a plane (X rows: within the planes of a
+    // work-group's at most 64 rows) have 32 bits
+    if ((double)sizeof(C2<T>) * Hp * (is2d ? N[1] : P[1]) * (2 + 64 / N[1]) >= 4294967296.0) return;
+    std::vector<C2<T>> h;
+    const int nx = P[0] / 2, ny = P[1], convlen = is2d ? P[1] : P[2];
+    if (!xodd && !CtTable<T>::x(nx) && !x4_ok<T>(nx, N[0])) rx.append(REG_X, nx, (long)N[1] * N[2], 3, roots, h);
+    if (!is2d && !coly_len<T>(ny)) ry.append(REG_COL, ny, H, 3L * N[2], roots, h);
+    rshort = !is2d && short_ok<T>(N[2], P[2]);
+    if (!rshort && !zreg && !CtTable<T>::conv(convlen, is2d, H))
+      rc.append(REG_CONV, convlen, H, is2d ? 1L : (long)P[1], roots, h);
+    if (h.empty()) return;
+    rtw.alloc(sizeof(C2<T>) * h.size());
+    UM_HIP(hipMemcpyAsync(rtw.p, h.data(), rtw.bytes, hipMemcpyHostToDevice, s));
+    UM_HIP(hipStreamSynchronize(s));
+    for (RegTab<T> *r : {&rx, &ry, &rc}) r->bind(rtw.as<C2<T>>());
+  }
+  static int log2i(int v) { int l = 0; while ((1 << l) < v) l++; return l; }
+
   // Transform the FP64 real-space tensor (device, 6 x P) into the stored
   // half spectrum of precision T.
   void load_kernel(double *const Kdev[6], hipStream_t s) {
     // FP64 FFT plan over the full padded box
     TwTable<double> dx, dx2, dy, dz;
-    dx.make(P[0] / 2, s);
-    dx2.make(P[0], s);
-    dy.make(P[1], s);
-    dz.make(P[2], s);
+    dx2.make(P[0], roots, s);
+    dx.make(P[0] / 2, roots, s);
+    dy.make(P[1], roots, s);
+    dz.make(P[2], roots, s);
     const int Hpd = (H + 7) / 8 * 8;
     DevBuf sp(sizeof(double2) * (size_t)P[2] * P[1] * Hpd);
     DevBuf mx(sizeof(unsigned long long));
@@ -2209,7 +1877,7 @@ struct DemagPlan : DemagBase {
         ca.f = dy.len; ca.nl = std::min(capd / P[1], 64); ca.fnl.init(ca.nl); ca.H = H; ca.nvalid = P[1]; ca.nout = P[1];
         ca.estride = Hpd; ca.pstride = (long)P[1] * Hpd; ca.buf[0] = (double2 *)sp.p;
         dim3 g((H + ca.nl - 1) / ca.nl, P[2], 1);
-        UM_LAUNCH((k_colfft<double, -1, 0, 0>), g, dim3(FFT_NT), sizeof(double2) * ca.nl * P[1], s, ca);
+        UM_LAUNCH((k_colfft<double, -1>), g, dim3(FFT_NT), sizeof(double2) * ca.nl * P[1], s, ca);
         UM_HIP(hipGetLastError());
       }
       if (P[2] > 1) {
@@ -2217,7 +1885,7 @@ struct DemagPlan : DemagBase {
         ca.f = dz.len; ca.nl = std::min(capd / P[2], 64); ca.fnl.init(ca.nl); ca.H = H; ca.nvalid = P[2]; ca.nout = P[2];
         ca.estride = (long)P[1] * Hpd; ca.pstride = Hpd; ca.buf[0] = (double2 *)sp.p;
         dim3 g((H + ca.nl - 1) / ca.nl, P[1], 1);
-        UM_LAUNCH((k_colfft<double, -1, 0, 0>), g, dim3(FFT_NT), sizeof(double2) * ca.nl * P[2], s, ca);
+        UM_LAUNCH((k_colfft<double, -1>), g, dim3(FFT_NT), sizeof(double2) * ca.nl * P[2], s, ca);
         UM_HIP(hipGetLastError());
       }
       UM_LAUNCH(k_extract_kspec<T>, dim3(blocks_for(kcount, 256, 4096)), dim3(256), 0, s,
@@ -2225,6 +1893,7 @@ struct DemagPlan : DemagBase {
                          (unsigned long long *)mx.p, zreg ? 1 : 0, c);
       UM_HIP(hipGetLastError());
     }
+    roots.tab.clear();
     unsigned long long bits = 0;
     UM_HIP(hipMemcpyAsync(&bits, mx.p, 8, hipMemcpyDeviceToHost, s));
     UM_HIP(hipStreamSynchronize(s));
@@ -2250,8 +1919,37 @@ struct DemagPlan : DemagBase {
       launch_b<BXfwdOdd<T>>(k_xfwd_odd<T>, g, dim3(FFT_NT), sizeof(C2<T>) * nl_x * P[0], s, a);
       UM_HIP(hipGetLastError());
     } else if (!(xi4 && launch_xf4<T>(a, P[0] / 2, s))) {
-      launch_xfwd<T>(a, P[0] / 2, nl_x, g, s);
+      if (rx.len.n && tx.sched == 0) {
+        RXArgs<T> r = rx_args();
+        r.in_pitch = Nx;
+        for (int c = 0; c < 3; c++) r.src[c] = (const T *)mv[c];
+        r.Ms = a.Ms; r.vol = a.vol;
+        r.pairs = even_pairs(r.src, a.Ms.arr, a.vol);
+        launch_rxfwd<T>(r, rx.nt, s);
+      } else {
+        launch_xfwd<T>(a, P[0] / 2, nl_x, g, s);
+      }
     }
+  }
+  // pairwise access to real rows: even Nx and every array aligned to two values
+  template <typename Q>
+  bool even_pairs(Q *const (&v)[3], const void *a, const void *b) const {
+    const uintptr_t bits = (uintptr_t)v[0] | (uintptr_t)v[1] | (uintptr_t)v[2] | (uintptr_t)a | (uintptr_t)b;
+    return N[0] % 2 == 0 && (bits & (2 * sizeof(T) - 1)) == 0;
+  }
+  RXArgs<T> rx_args() const {
+    RXArgs<T> r{};
+    r.f = rx.len; r.tw2 = (const C2<T> *)tx2.buf.p; r.nl = rx.nl; r.Nx = N[0]; r.rows = N[1] * N[2];
+    r.Py = is2d ? N[1] : P[1]; r.Hp = Hp; r.fhalf.init(P[0] / 4 + 1); r.fRy.init(N[1]);
+    for (int c = 0; c < 3; c++) r.spec[c] = spec[c].template as<C2<T>>();
+    return r;
+  }
+  void rcol(int dir, hipStream_t s) {
+    RColArgs<T> a{};
+    a.f = ry.len; a.lsh = log2i(ry.nl); a.H = H; a.nvalid = dir < 0 ? N[1] : P[1]; a.nout = dir < 0 ? P[1] : N[1];
+    a.estride = Hp; a.pstride = (long)P[1] * Hp;
+    for (int c = 0; c < 3; c++) a.buf[c] = spec[c].template as<C2<T>>();
+    launch_rcol<T>(a, dir, N[2], ry.nt, s);
   }
   // Y forward (dir < 0) or inverse (dir > 0), 3D only
   void pass_y(int dir, hipStream_t s) {
@@ -2261,10 +1959,14 @@ struct DemagPlan : DemagBase {
     dim3 gy((H + nl_y - 1) / nl_y, N[2], 3);
     if (dir < 0) {
       ya.nvalid = N[1]; ya.nout = P[1];
-      if (!launch_coly<T, -1>(ya, P[1], N[2], s)) launch_col<T, -1>(ya, P[1], nl_y, gy, s);
+      if (launch_coly<T, -1>(ya, P[1], N[2], s)) return;
+      if (ry.len.n && ty.sched == 0) rcol(dir, s);
+      else launch_col<T, -1>(ya, P[1], nl_y, gy, s);
     } else {
       ya.nvalid = P[1]; ya.nout = N[1];
-      if (!launch_coly<T, +1>(ya, P[1], N[2], s)) launch_col<T, +1>(ya, P[1], nl_y, gy, s);
+      if (launch_coly<T, +1>(ya, P[1], N[2], s)) return;
+      if (ry.len.n && ty.sched == 0) rcol(dir, s);
+      else launch_col<T, +1>(ya, P[1], nl_y, gy, s);
     }
   }
   // the convolution pass: Z (3D) or Y (2D) forward, tensor multiply, inverse
@@ -2278,6 +1980,24 @@ struct DemagPlan : DemagBase {
       za.K = kern.as<T>();
       for (int c = 0; c < 3; c++) za.buf[c] = spec[c].as<C2<T>>();
       launch_convz<T>(za, N[2], s);
+      return;
+    }
+    if (rshort && tz.sched == 0) {
+      RShortArgs<T> r{};
+      r.H = H; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk; r.zstride = (long)P[1] * Hp; r.ystride = Hp;
+      for (int c = 0; c < 6; c++) r.K[c] = K[c];
+      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>();
+      launch_rshort<T>(r, N[2], s);
+      return;
+    }
+    if (rc.len.n && (is2d ? ty : tz).sched == 0) {
+      RConvArgs<T> r{};
+      r.f = rc.len; r.lsh = log2i(rc.nl); r.H = H; r.nvalid = is2d ? N[1] : N[2];
+      r.estride = is2d ? Hp : (long)P[1] * Hp; r.pstride = is2d ? 0 : Hp;
+      r.is2d = is2d; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk;
+      for (int c = 0; c < 6; c++) r.K[c] = K[c];
+      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>();
+      launch_rconv<T>(r, rc.nt, s);
       return;
     }
     ConvArgs<T> ca{};
@@ -2306,8 +2026,15 @@ struct DemagPlan : DemagBase {
       a.f = tx2.len; a.fhalf.init(H);
       launch_b<BXinvOdd<T>>(k_xinv_odd<T>, g, dim3(FFT_NT), sizeof(C2<T>) * nl_xi * P[0], s, a);
       UM_HIP(hipGetLastError());
-    } else {
-      launch_xinv<T>(a, P[0] / 2, nl_xi, g, s, xi4);
+    } else if (!(xi4 && launch_xi4<T>(a, P[0] / 2, s))) {
+      if (rx.len.n && tx.sched == 0) {
+        RXArgs<T> r = rx_args();
+        for (int c = 0; c < 3; c++) r.dst[c] = (T *)Bv[c];
+        r.pairs = even_pairs(r.dst, nullptr, nullptr);
+        launch_rxinv<T>(r, rx.nt, s);
+      } else {
+        launch_xinv<T>(a, P[0] / 2, nl_xi, g, s, false);
+      }
     }
   }
 
@@ -2470,7 +2197,6 @@ struct DemagPlan : DemagBase {
       if (!is2d) {
         std::vector<int> nls;
         add(nls, nl_y);
-        add(nls, CtTable<T>::col(P[1]));
         for (int x : halvings(std::min(lines_for(P[1]), 64))) add(nls, x);
         float best = 1e30f;
         int bn = nl_y, bs = ty.sched;
@@ -2490,9 +2216,7 @@ struct DemagPlan : DemagBase {
         const int convlen = is2d ? P[1] : P[2];
         std::vector<int> bs_;
         add(bs_, B_conv);
-        const int ct = is2d ? CtTable<T>::conv2(convlen) : CtTable<T>::conv3(convlen);
-        add(bs_, ct);
-        add(bs_, ct / 4);
+        add(bs_, CtTable<T>::conv(convlen, is2d, H));
         for (int x : halvings(std::min(lines_for(convlen) / 3, 32))) add(bs_, x);
         float best = 1e30f;
         int bb_ = B_conv, bsc = tc.sched;

@@ -1,0 +1,10 @@
+// FP64 register-stage passes.
+#include <cmath>
+
+#include "demag_reg_kernels.hpp"
+
+namespace um {
+
+UM_REG_INSTANTIATE(double)
+
+}  // namespace um

@@ -162,13 +162,62 @@ __device__ __forceinline__ void dft_odd(C *a) {
   for (int j = 0; j < R; j++) a[j] = out[j];
 }
 template <int R, int DIR, typename C>
+__device__ __forceinline__ void dft(C *a);
+// exp(dir * 2 pi i j / n); constant once the caller's loops are unrolled
+template <typename T>
+__device__ __forceinline__ C2<T> cexpi(int j, int n, int dir) {
+  const double ang = 2.0 * M_PI * (double)j / (double)n;
+  return C2<T>{T(__builtin_cos(ang)), T(dir * __builtin_sin(ang))};
+}
+// R = A B in registers (Cooley-Tukey, compile-time twiddles): B-point
+// transforms of the A interleaved subsequences, then A-point ones
+template <int A, int B, int DIR, typename C>
+__device__ __forceinline__ void dft_ab(C *a) {
+  using S = decltype(a[0].x);
+  C t[A][B];
+#pragma unroll
+  for (int p = 0; p < A; p++) {
+#pragma unroll
+    for (int q = 0; q < B; q++) t[p][q] = a[p + A * q];
+    dft<B, DIR>(t[p]);
+#pragma unroll
+    for (int k = 1; k < B; k++)
+      if (p > 0) t[p][k] = cmul(t[p][k], cexpi<S>(p * k, A * B, DIR));
+  }
+#pragma unroll
+  for (int k = 0; k < B; k++) {
+    C u[A];
+#pragma unroll
+    for (int p = 0; p < A; p++) u[p] = t[p][k];
+    dft<A, DIR>(u);
+#pragma unroll
+    for (int j = 0; j < A; j++) a[k + B * j] = u[j];
+  }
+}
+template <int R, int DIR, typename C>
 __device__ __forceinline__ void dft(C *a) {
-  if constexpr (R == 2) dft2<DIR>(a[0], a[1]);
+  if constexpr (R == 1) return;
+  else if constexpr (R == 2) dft2<DIR>(a[0], a[1]);
   else if constexpr (R == 4) dft4<DIR>(a[0], a[1], a[2], a[3]);
+  else if constexpr (R == 6) dft_ab<2, 3, DIR>(a);
   else if constexpr (R == 8) dft8<DIR>(a);
+  else if constexpr (R == 9) dft_ab<3, 3, DIR>(a);
+  else if constexpr (R == 10) dft_ab<2, 5, DIR>(a);
+  else if constexpr (R == 12) dft_ab<4, 3, DIR>(a);
+  else if constexpr (R == 14) dft_ab<2, 7, DIR>(a);
+  else if constexpr (R == 15) dft_ab<3, 5, DIR>(a);
   else if constexpr (R == 16) dft16<DIR>(a);
+  else if constexpr (R == 20) dft_ab<4, 5, DIR>(a);
   else if constexpr (R == 32) dft32<DIR>(a);
   else dft_odd<R, DIR>(a);
+}
+
+// Work-group index permuted so that the tiles one XCD runs (linear ids w,
+// w+8, w+16, ... are dispatched to the same XCD) are adjacent in memory and
+// share their 128-byte lines in that XCD's L2.
+__device__ __forceinline__ int xcd_tile(int w, int total) {
+  const int q = total >> 3, full = q << 3;
+  return w >= full ? w : (w & 7) * q + (w >> 3);
 }
 
 // ---- register-level helpers ------------------------------------------------
