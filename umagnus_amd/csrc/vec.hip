@@ -273,13 +273,49 @@ __device__ __forceinline__ void block_max_to(double v, unsigned long long *dst) 
   __syncthreads();
 }
 
+// three maxima of a work-group of up to 16 waves into dst[0..n-1] (NaN wins):
+// one barrier, and one atomic per slot issued by lanes of the same wave
+template <int N>
+__device__ __forceinline__ void block_max_n(const double (&v)[N], unsigned long long *dst) {
+  __shared__ double sh[N][16];
+  const int w = threadIdx.x / 64, l = threadIdx.x % 64, nw = (int)(blockDim.x + 63) / 64;
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const double m = wave_max(v[i]);
+    if (l == 0) sh[i][w] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x < N) {
+    double m = sh[threadIdx.x][0];
+    for (int i = 1; i < nw; i++) m = nmax(m, sh[threadIdx.x][i]);
+    if (m != m) m = __longlong_as_double(0x7ff8000000000000LL);
+    atomicMax(dst + threadIdx.x, (unsigned long long)__double_as_longlong(m));
+  }
+}
+// running maximum of |E| / |k7| as the pair of squares with the largest
+// quotient (compared by cross products): one division per thread instead of
+// two square roots and a division per cell in FP64.  Products near the ends of
+// the range compare the quotients themselves.  A pair with k7 = 0 counts as 0
+// (div.cl:9), one with a NaN is skipped.
+struct RelMax {
+  double e2 = 0, k2 = 1;
+  __device__ __forceinline__ void add(double e, double k) {
+    const double p = e * k2, q = e2 * k, big = fmax(p, q);
+    bool more = p > q;
+    if (!(big > 1e-280 && big < 1e300)) more = sqrt(e) / sqrt(k) > sqrt(e2) / sqrt(k2);
+    if (k != 0.0 && more) { e2 = e; k2 = k; }
+  }
+  __device__ __forceinline__ double value() const { return sqrt(e2) / sqrt(k2); }
+};
+
 // ---- fused error reductions --------------------------------------------------------
 template <typename T>
 struct BErr {
   using Args = ErrArgs<T>;
   static constexpr int NT = 256, MINB = 1;
   static __device__ __forceinline__ void run(const ErrArgs<T> &a, uint3 blockIdx, uint3 gridDim) {
-    double m0 = 0, m1 = 0, m2 = 0;
+    double m0 = 0, m1 = 0;
+    RelMax rel;
     bool nan = false;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.N; i += (long)gridDim.x * blockDim.x) {
       if (a.mode == 0) {
@@ -296,11 +332,10 @@ struct BErr {
         const double e2 = (double)E[0] * E[0] + (double)E[1] * E[1] + (double)E[2] * E[2];
         const double k2 = (double)K7[0] * K7[0] + (double)K7[1] * K7[1] + (double)K7[2] * K7[2];
         // VecNorm(errnorm)/VecNorm(ddtnorm), 0 where |k7| = 0 (div.cl:9)
-        const double rel = (k2 == 0.0) ? 0.0 : sqrt(e2) / sqrt(k2);
+        rel.add(e2, k2);
         nan |= (e2 != e2);
         m0 = fmax(m0, e2);
         m1 = fmax(m1, k2);
-        m2 = fmax(m2, rel);
       } else if (a.mode == 1) {
         const double dx = (double)(a.k[0][0][i] - a.k[1][0][i]);
         const double dy = (double)(a.k[0][1][i] - a.k[1][1][i]);
@@ -316,10 +351,11 @@ struct BErr {
       }
     }
     if (nan) m0 = __longlong_as_double(0x7ff8000000000000LL);
-    block_max_to(m0, a.res);
     if (a.mode == 0) {
-      block_max_to(m1, a.res + 1);
-      block_max_to(m2, a.res + 2);
+      const double v[3] = {m0, m1, rel.value()};
+      block_max_n(v, a.res);
+    } else {
+      block_max_to(m0, a.res);
     }
   }
 };
@@ -333,10 +369,10 @@ struct BErrV {
   static __device__ __forceinline__ void run(const ErrArgs<T> &a, uint3 blockIdx, uint3 gridDim) {
     using V = typename Vec16<T>::type;
     constexpr int W = Vec16<T>::n, NK = MODE == 0 ? 6 : MODE == 1 ? 2 : 1;
-    double m0 = 0, m1 = 0, m2 = 0;
+    double m0 = 0, m1 = 0;
+    RelMax rel;
     bool nan = false;
     const long groups = a.N / W;
-  #pragma unroll 2
     for (long g = blockIdx.x * 256L + threadIdx.x; g < groups; g += (long)gridDim.x * 256) {
       T x[NK][3][W];
   #pragma unroll
@@ -360,12 +396,11 @@ struct BErrV {
           const double e2 = (double)E[0] * E[0] + (double)E[1] * E[1] + (double)E[2] * E[2];
           const double k2 = (double)x[5][0][w] * x[5][0][w] + (double)x[5][1][w] * x[5][1][w] +
                             (double)x[5][2][w] * x[5][2][w];
-          const double rel = (k2 == 0.0) ? 0.0 : sqrt(e2) / sqrt(k2);
+          rel.add(e2, k2);
           nan |= (e2 != e2);
           m0 = fmax(m0, e2);
           m1 = fmax(m1, k2);
-          m2 = fmax(m2, rel);
-        } else if (MODE == 1) {
+          } else if (MODE == 1) {
           const double dx = (double)(x[0][0][w] - x[1][0][w]);
           const double dy = (double)(x[0][1][w] - x[1][1][w]);
           const double dz = (double)(x[0][2][w] - x[1][2][w]);
@@ -381,10 +416,11 @@ struct BErrV {
       }
     }
     if (nan) m0 = __longlong_as_double(0x7ff8000000000000LL);
-    block_max_to(m0, a.res);
-    if (MODE == 0) {
-      block_max_to(m1, a.res + 1);
-      block_max_to(m2, a.res + 2);
+    if constexpr (MODE == 0) {
+      const double v[3] = {m0, m1, rel.value()};
+      block_max_n(v, a.res);
+    } else {
+      block_max_to(m0, a.res);
     }
   }
 };
@@ -399,17 +435,19 @@ void launch_err(const ErrArgs<T> &a, hipStream_t s) {
   for (int j = 0; j < nk && vec; j++)
     for (int c = 0; c < 3; c++) vec = vec && ((uintptr_t)a.k[j][c] & 15) == 0;
   if (vec) {
-    // at most 512 work-groups: each ends with three device-scope atomic maxima
-    // on the same three slots, which serialise (2048 work-groups: 124 us at
-    // 8.4M cells, 512: 114 us)
-    const dim3 grid(blocks_for(a.N / W, 256, 512));
+    // at most one work-group a CU: each ends with a device-scope atomic maximum
+    // per slot, which serialise, and four waves a CU with 18 loads each in
+    // flight reach the copy rate (RK45DP, 8.4M cells FP32: 101 us with 256
+    // work-groups, 109 with 1024, 119 with 128; 524k cells: 14 us, against 23
+    // with three separate atomics for each of 512 and a square root per cell)
+    const dim3 grid(blocks_for(a.N / W, 256, 256));
     if (a.mode == 0) launch_b<BErrV<T, 0>>(k_err_v<T, 0>, grid, dim3(256), 0, s, a);
     else if (a.mode == 1) launch_b<BErrV<T, 1>>(k_err_v<T, 1>, grid, dim3(256), 0, s, a);
     else launch_b<BErrV<T, 2>>(k_err_v<T, 2>, grid, dim3(256), 0, s, a);
     UM_HIP(hipGetLastError());
     return;
   }
-  launch_b<BErr<T>>(k_err<T>, dim3(blocks_for(a.N, 256, 2048)), dim3(256), 0, s, a);
+  launch_b<BErr<T>>(k_err<T>, dim3(blocks_for(a.N, 256, 512)), dim3(256), 0, s, a);
   UM_HIP(hipGetLastError());
 }
 template void launch_err<float>(const ErrArgs<float> &, hipStream_t);
