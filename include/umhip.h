@@ -452,10 +452,10 @@ int um_sim_kernel_times(void *sim, double out_ms[3], int *n_evals);
 
 /* ---- HIP graphs and ensembles (no counterpart in the reference, whose steps
  * are enqueued call by call) ------------------------------------------------ */
-/* With FixDt set, um_sim_steps runs one step eagerly, then replays a captured
- * two-step HIP graph (no host synchronisation per step: the step statistics
- * and the thermal Philox step counter stay on the device) and reads the
- * statistics back once.  Results are identical to eager stepping.  The graph
+/* With FixDt set, um_sim_steps replays a captured two-step HIP graph (no host
+ * synchronisation per step: the step statistics and the thermal Philox step
+ * counter stay on the device), reads the statistics back once and runs an odd
+ * last step eagerly.  Results are identical to eager stepping.  The graph
  * is re-captured after any parameter or solver change.  Adaptive steps
  * (FixDt = 0) always run eagerly. */
 int um_sim_set_graph(void *sim, int on);
@@ -467,12 +467,13 @@ int um_sim_set_graph(void *sim, int on);
 int um_sims_steps(int nsims, void *const *sims, int n);
 /* Ensemble stepping in batched launches, the one-launch form of the same job
  * queue (cmd/uMagNUS/queue.go:86-151): n steps of every simulation in sims[]
- * (each handle once).  After one eager step per member, the launches of two
- * fixed-dt steps of every member in graph mode are recorded and merged: each
- * kernel variant runs once per phase for all members that reach it, every
+ * (each handle once).  The launches of two fixed-dt
+ * steps of every member in graph mode are recorded and merged: each kernel
+ * variant runs once per phase for all members that reach it (large ensembles:
+ * for the members of each of a few chains that run side by side), every
  * work-group working on its own member's grid and buffers, so each member
  * computes what it computes alone (um_sims_steps, um_sim_steps), bit for bit.
- * The merged sequence is replayed as one graph per two steps; it is rebuilt
+ * The merged sequences are replayed as graphs of two steps; they are rebuilt
  * when a member's parameters, solver, FixDt or buffers change.  Members not in
  * graph mode with FixDt step eagerly in turn.  *launches_per_two_steps (when
  * not NULL) receives the number of launches that replay two steps of the

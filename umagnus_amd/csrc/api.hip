@@ -1094,11 +1094,14 @@ int um_sims_steps(int nsims, void *const *sims, int n) {
 
 // ---- batched ensembles -----------------------------------------------------------------
 // The recorded two-step launch lists of the members, merged into batched
-// launches: phase by phase, the kernel family that most members have next runs
-// for all of them (one k_batch launch per distinct kernel variant), each
-// member's launches keeping their order.  The tables (arguments, work-group
-// prefix, member grids) live in one device buffer; the launch sequence is
-// captured once into a graph on the plan's stream.
+// launches: phase by phase, a kernel family runs for all members that have
+// reached it once those that still have it ahead in the same part of the step
+// have too (one k_batch launch per distinct kernel variant), each member's
+// launches keeping their order.  The tables (arguments, work-group
+// prefix, member grids) live in one device buffer.  The members are dealt to
+// up to BATCH_CHAINS chains, members with the same kernels together; a chain is
+// one launch sequence, captured once into a graph and replayed on a stream of
+// its own, so the partly filled launches of different chains overlap.
 namespace um {
 struct BatchGroupLaunch {
   void (*launch)(const void *, const uint32_t *, const uint3 *, int, unsigned, dim3, size_t, hipStream_t);
@@ -1108,22 +1111,37 @@ struct BatchGroupLaunch {
   dim3 block;
   size_t lds;
 };
-struct BatchPlan {
-  std::vector<const void *> sims;
-  std::vector<std::vector<uint64_t>> keys;
+// HIP maps streams onto four hardware queues by default; a chain should have
+// enough members to share its launches.  48 thermal Heun members of 32..256
+// cells a side, 20 steps: 20.5 ms in one chain (140 launches per two steps),
+// 16.7 in two, 15.3 in three, 15.1 in four (328)
+constexpr int BATCH_CHAINS = 4, BATCH_CHAIN_MEMBERS = 12;
+struct BatchChain {
+  std::vector<int> members;
   std::vector<BatchGroupLaunch> launches;
-  DevBuf tab;
   hipStream_t st = nullptr;
   hipGraphExec_t gexec = nullptr;
   hipEvent_t done = nullptr;
+};
+struct BatchPlan {
+  std::vector<const void *> sims;
+  std::vector<std::vector<uint64_t>> keys;
+  std::vector<BatchChain> chains;
+  DevBuf tab;
   std::vector<hipEvent_t> ready;
-  int launches_per_replay() const { return (int)launches.size(); }
+  int launches_per_replay() const {
+    size_t n = 0;
+    for (const BatchChain &c : chains) n += c.launches.size();
+    return (int)n;
+  }
   ~BatchPlan() {
-    if (st) (void)hipStreamSynchronize(st);
-    if (gexec) (void)hipGraphExecDestroy(gexec);
+    for (BatchChain &c : chains) {
+      if (c.st) (void)hipStreamSynchronize(c.st);
+      if (c.gexec) (void)hipGraphExecDestroy(c.gexec);
+      if (c.done) (void)hipEventDestroy(c.done);
+      if (c.st) (void)hipStreamDestroy(c.st);
+    }
     for (hipEvent_t e : ready) (void)hipEventDestroy(e);
-    if (done) (void)hipEventDestroy(done);
-    if (st) (void)hipStreamDestroy(st);
   }
 };
 static std::mutex g_bmu;
@@ -1154,6 +1172,28 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
       auto it = famid.emplace(body_family(e.fam), (int)famid.size()).first;
       fam[i].push_back(it->second);
     }
+  // members with equal kernel sequences next to each other, cut into chains of
+  // about equal work (threads launched)
+  std::vector<std::vector<std::pair<const void *, unsigned>>> sig(nm);
+  std::vector<double> cost(nm, 0.0);
+  double all = 0;
+  for (int i = 0; i < nm; i++) {
+    for (const BatchEntry &e : rec[i]) {
+      sig[i].emplace_back(e.key, e.block.x);
+      cost[i] += (double)e.grid.x * e.grid.y * e.grid.z * e.block.x;
+    }
+    all += cost[i];
+  }
+  std::vector<int> order(nm);
+  for (int i = 0; i < nm; i++) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sig[a] < sig[b]; });
+  const int nc = std::max(1, std::min(BATCH_CHAINS, nm / BATCH_CHAIN_MEMBERS));
+  P->chains.resize(nc);
+  double before = 0;
+  for (int i : order) {
+    P->chains[std::min(nc - 1, (int)((before + 0.5 * cost[i]) * nc / all))].members.push_back(i);
+    before += cost[i];
+  }
   std::vector<size_t> head(nm, 0);
   std::vector<unsigned char> host;
   auto put = [&](const void *p, size_t bytes) {
@@ -1162,23 +1202,53 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
     std::memcpy(host.data() + off, p, bytes);
     return off;
   };
+  for (BatchChain &ch : P->chains) {
+  // families that every member of the chain launches equally often (stages,
+  // norms, statistics) cut the lists into segments
+  std::vector<char> anchor(famid.size(), 1);
+  {
+    std::vector<std::vector<int>> n(ch.members.size(), std::vector<int>(famid.size(), 0));
+    for (size_t c = 0; c < ch.members.size(); c++) {
+      for (int f : fam[ch.members[c]]) n[c][f]++;
+      for (size_t f = 0; f < famid.size(); f++) anchor[f] = anchor[f] && n[c][f] > 0 && n[c][f] == n[0][f];
+    }
+  }
   for (;;) {
-    std::vector<int> count(famid.size(), 0);
+    // members at each family, and those that still meet it in their segment; a
+    // family is launched when all of these are at it, an anchor last
+    std::vector<int> at(famid.size(), 0), due(famid.size(), 0);
     bool any = false;
-    for (int i = 0; i < nm; i++)
-      if (head[i] < rec[i].size()) { count[fam[i][head[i]]]++; any = true; }
+    for (int i : ch.members) {
+      if (head[i] >= rec[i].size()) continue;
+      any = true;
+      at[fam[i][head[i]]]++;
+      std::vector<char> seen(famid.size(), 0);
+      for (size_t h = head[i]; h < rec[i].size(); h++) {
+        const int f = fam[i][h];
+        if (!seen[f]) { seen[f] = 1; due[f]++; }
+        if (anchor[f]) break;
+      }
+    }
     if (!any) break;
-    const int f = (int)(std::max_element(count.begin(), count.end()) - count.begin());
+    int f = -1;
+    auto better = [&](int a, int b) {   // a before b
+      if (b < 0) return true;
+      if (anchor[a] != anchor[b]) return !anchor[a];
+      if ((at[a] == due[a]) != (at[b] == due[b])) return at[a] == due[a];
+      return at[a] > at[b];
+    };
+    for (int c = 0; c < (int)famid.size(); c++)
+      if (at[c] > 0 && better(c, f)) f = c;
     // members whose next launch is of family f, grouped by kernel variant
     std::vector<std::pair<const BatchEntry *, std::vector<int>>> groups;
-    for (int i = 0; i < nm; i++) {
+    for (int i : ch.members) {
       if (head[i] >= rec[i].size() || fam[i][head[i]] != f) continue;
       const BatchEntry &e = rec[i][head[i]++];
       bool placed = false;
       for (auto &g : groups) {
         const BatchEntry &r = *g.first;
-        if (r.key == e.key && r.lds == e.lds && r.block.x == e.block.x && r.block.y == e.block.y &&
-            r.block.z == e.block.z) {
+        // dynamic LDS may differ: the launch takes the largest
+        if (r.key == e.key && r.block.x == e.block.x && r.block.y == e.block.y && r.block.z == e.block.z) {
           g.second.push_back(i);
           placed = true;
           break;
@@ -1193,6 +1263,7 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
       std::vector<uint32_t> start(gn);
       std::vector<uint3> grid(gn);
       unsigned long long total = 0;
+      size_t lds = 0;
       for (int j = 0; j < gn; j++) {
         const int i = g.second[j];
         const BatchEntry &e = rec[i][head[i] - 1];
@@ -1200,6 +1271,7 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
         start[j] = (uint32_t)total;
         grid[j] = make_uint3(e.grid.x, e.grid.y, e.grid.z);
         total += (unsigned long long)e.grid.x * e.grid.y * e.grid.z;
+        lds = std::max(lds, e.lds);
       }
       UM_REQUIRE(total > 0 && total < (1ull << 31), UM_EUNSUP, "batched launch too large");
       BatchGroupLaunch L;
@@ -1210,34 +1282,37 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
       L.nm = gn;
       L.total = (unsigned)total;
       L.block = r.block;
-      L.lds = r.lds;
-      P->launches.push_back(L);
+      L.lds = lds;
+      ch.launches.push_back(L);
     }
+  }
   }
   P->tab.alloc(std::max<size_t>(host.size(), 256));
   UM_HIP(hipMemcpy(P->tab.p, host.data(), host.size(), hipMemcpyHostToDevice));
-  UM_HIP(hipStreamCreateWithFlags(&P->st, hipStreamNonBlocking));
-  UM_HIP(hipEventCreateWithFlags(&P->done, hipEventDisableTiming));
   P->ready.resize(nm);
   for (int i = 0; i < nm; i++) UM_HIP(hipEventCreateWithFlags(&P->ready[i], hipEventDisableTiming));
-  // the replay: every batched launch in order, captured once
+  // the replays: each chain's launches in order, captured once
   const unsigned char *base = (const unsigned char *)P->tab.p;
-  hipGraph_t g = nullptr;
-  UM_HIP(hipStreamBeginCapture(P->st, hipStreamCaptureModeRelaxed));
-  try {
-    for (const BatchGroupLaunch &L : P->launches)
-      L.launch(base + L.a_off, (const uint32_t *)(base + L.s_off), (const uint3 *)(base + L.g_off), L.nm, L.total,
-               L.block, L.lds, P->st);
-  } catch (...) {
-    hipGraph_t junk = nullptr;
-    (void)hipStreamEndCapture(P->st, &junk);
-    if (junk) (void)hipGraphDestroy(junk);
-    throw;
+  for (BatchChain &ch : P->chains) {
+    UM_HIP(hipStreamCreateWithFlags(&ch.st, hipStreamNonBlocking));
+    UM_HIP(hipEventCreateWithFlags(&ch.done, hipEventDisableTiming));
+    hipGraph_t g = nullptr;
+    UM_HIP(hipStreamBeginCapture(ch.st, hipStreamCaptureModeRelaxed));
+    try {
+      for (const BatchGroupLaunch &L : ch.launches)
+        L.launch(base + L.a_off, (const uint32_t *)(base + L.s_off), (const uint3 *)(base + L.g_off), L.nm, L.total,
+                 L.block, L.lds, ch.st);
+    } catch (...) {
+      hipGraph_t junk = nullptr;
+      (void)hipStreamEndCapture(ch.st, &junk);
+      if (junk) (void)hipGraphDestroy(junk);
+      throw;
+    }
+    UM_HIP(hipStreamEndCapture(ch.st, &g));
+    hipError_t e = hipGraphInstantiate(&ch.gexec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    UM_HIP(e);
   }
-  UM_HIP(hipStreamEndCapture(P->st, &g));
-  hipError_t e = hipGraphInstantiate(&P->gexec, g, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(g);
-  UM_HIP(e);
   return P.release();
 }
 
@@ -1287,16 +1362,20 @@ int um_sims_steps_batched(int nsims, void *const *sims, int n, int *launches_per
       if (batched) {
         BatchPlan *P = g_bplan;
         g_batch_launches = P->launches_per_replay();
-        for (size_t i = 0; i < mem.size(); i++) {
-          UM_HIP(hipEventRecord(P->ready[i], mem[i]->stream()));
-          UM_HIP(hipStreamWaitEvent(P->st, P->ready[i], 0));
-        }
+        for (BatchChain &ch : P->chains)
+          for (int i : ch.members) {
+            UM_HIP(hipEventRecord(P->ready[i], mem[i]->stream()));
+            UM_HIP(hipStreamWaitEvent(ch.st, P->ready[i], 0));
+          }
         for (long r = 0; r < R; r++) {
-          UM_HIP(hipGraphLaunch(P->gexec, P->st));
+          for (BatchChain &ch : P->chains)
+            if (ch.gexec) UM_HIP(hipGraphLaunch(ch.gexec, ch.st));
           for (SimBase *x : mem) x->batch_advance();
         }
-        UM_HIP(hipEventRecord(P->done, P->st));
-        for (SimBase *x : mem) UM_HIP(hipStreamWaitEvent(x->stream(), P->done, 0));
+        for (BatchChain &ch : P->chains) {
+          UM_HIP(hipEventRecord(ch.done, ch.st));
+          for (int i : ch.members) UM_HIP(hipStreamWaitEvent(mem[i]->stream(), ch.done, 0));
+        }
       } else {
         g_batch_launches = 0;
         for (SimBase *x : mem) x->graph_ensure();

@@ -490,6 +490,16 @@ struct Sim : SimBase {
     }
     return a;
   }
+  // the masked demag input of NoDemagSpins, when a parameter changed
+  void nodemag_input() {
+    if (nd_gen == gen && ndvol.p) return;
+    if (!ndvol.p) ndvol.alloc(sizeof(T) * n);
+    UM_LAUNCH(k_nodemag_vol<T>, dim3(blocks_for(n, 256, 8192)), dim3(256), 0, st, ndvol.as<T>(),
+                       (const T *)vol.p, nodemagLUT.as<T>(), has_regions ? (const uint8_t *)regions.p : nullptr,
+                       (long)n);
+    UM_HIP(hipGetLastError());
+    nd_gen = gen;
+  }
   // B_demag into bd (SetDemagField, engine/demag.go:42-65); with NoDemagSpins
   // the flagged cells neither generate nor receive the field (:67-98)
   void compute_demag(const T *mm) {
@@ -499,14 +509,7 @@ struct Sim : SimBase {
     const void *mv[3] = {mm, mm + n, mm + 2 * n};
     const void *v = vol.p;
     if (has_nodemag) {
-      if (nd_gen != gen || !ndvol.p) {
-        if (!ndvol.p) ndvol.alloc(sizeof(T) * n);
-        UM_LAUNCH(k_nodemag_vol<T>, dim3(blocks_for(n, 256, 8192)), dim3(256), 0, st, ndvol.as<T>(),
-                           (const T *)vol.p, nodemagLUT.as<T>(), has_regions ? (const uint8_t *)regions.p : nullptr,
-                           (long)n);
-        UM_HIP(hipGetLastError());
-        nd_gen = gen;
-      }
+      nodemag_input();
       v = ndvol.p;
     }
     demag_exec(demag, B, mv, v, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul, st);
@@ -1189,8 +1192,8 @@ struct Sim : SimBase {
   bool graph_usable() const {
     return graph_mode && fixdt != 0 && !profiling && !tape_on && !any_tfn && !xterm_tfn;
   }
-  // one eager step (FSAL setup), then capture two steps if the cached graph is
-  // stale; returns how many two-step replays fit before `stop`
+  // the FSAL torque, then capture two steps if the cached graph is stale;
+  // returns how many two-step replays fit before `stop`
   // Every Steps/RunWhile starts without the FSAL torque (engine/run.go:207,
   // stepper.Free()), so the ensemble entry point and Steps agree
   long graph_prepare(long stop) override { return prepare_replays(stop, true); }
@@ -1204,11 +1207,22 @@ struct Sim : SimBase {
   long prepare_replays(long stop, bool capture) {
     k1_valid = false;
     if (!graph_usable() || nsteps >= stop) return 0;
-    step();
     if (nsteps + 2 > stop) return 0;
+    // A captured step computes what an eager one does, so the replays may start
+    // at once: they need the plan, the FSAL torque of the solvers that keep one,
+    // and what is otherwise prepared at the first evaluation.
+    ensure_demag();
+    dt = fixdt;
+    if (has_nodemag) nodemag_input();
+    if (!xterms.empty()) field_args(m);
     const void *ptrs[8] = {m, m0, k[0], k[1], k[2], k[3], k[4], k[5]};
     bool fresh = gexec && g_gen == gen && g_solver == solver && g_dt == fixdt;
     for (int i = 0; i < 8 && fresh; i++) fresh = (g_ptrs[i] == ptrs[i]);
+    if (capture && !fresh && nsteps + 3 > stop) return 0;   // two steps do not pay for a capture
+    if (!k1_valid && (solver == UM_SOLVER_RK45DP || solver == UM_SOLVER_RK23)) {
+      torque_fn(k[0]);
+      k1_valid = true;
+    }
     if (capture && !fresh) capture2();
     fill_bytes(red.p, red.bytes, st);   // the replays' reductions start from cleared slots
     hstat[0] = lastErr; hstat[1] = peakErr; hstat[2] = lastTorque;
