@@ -1944,79 +1944,101 @@ struct DemagPlan : DemagBase {
     for (int c = 0; c < 3; c++) r.spec[c] = spec[c].template as<C2<T>>();
     return r;
   }
-  void rcol(int dir, hipStream_t s) {
+  struct Cols { int x0, n; };   // kx columns of a pass
+  void rcol(int dir, Cols k, hipStream_t s) {
     RColArgs<T> a{};
-    a.f = ry.len; a.lsh = log2i(ry.nl); a.H = H; a.nvalid = dir < 0 ? N[1] : P[1]; a.nout = dir < 0 ? P[1] : N[1];
+    a.f = ry.len; a.lsh = log2i(ry.nl); a.H = k.n; a.nvalid = dir < 0 ? N[1] : P[1]; a.nout = dir < 0 ? P[1] : N[1];
     a.estride = Hp; a.pstride = (long)P[1] * Hp;
-    for (int c = 0; c < 3; c++) a.buf[c] = spec[c].template as<C2<T>>();
+    for (int c = 0; c < 3; c++) a.buf[c] = spec[c].template as<C2<T>>() + k.x0;
     launch_rcol<T>(a, dir, N[2], ry.nt, s);
   }
   // Y forward (dir < 0) or inverse (dir > 0), 3D only
-  void pass_y(int dir, hipStream_t s) {
+  void pass_y(int dir, Cols k, hipStream_t s) {
     ColArgs<T> ya{};
-    ya.f = ty.len; ya.nl = nl_y; ya.fnl.init(nl_y); ya.H = H; ya.estride = Hp; ya.pstride = (long)P[1] * Hp;
-    for (int c = 0; c < 3; c++) ya.buf[c] = spec[c].as<C2<T>>();
-    dim3 gy((H + nl_y - 1) / nl_y, N[2], 3);
+    ya.f = ty.len; ya.nl = nl_y; ya.fnl.init(nl_y); ya.H = k.n; ya.estride = Hp; ya.pstride = (long)P[1] * Hp;
+    for (int c = 0; c < 3; c++) ya.buf[c] = spec[c].as<C2<T>>() + k.x0;
+    dim3 gy((k.n + nl_y - 1) / nl_y, N[2], 3);
     if (dir < 0) {
       ya.nvalid = N[1]; ya.nout = P[1];
       if (launch_coly<T, -1>(ya, P[1], N[2], s)) return;
-      if (ry.len.n && ty.sched == 0) rcol(dir, s);
+      if (ry.len.n && ty.sched == 0) rcol(dir, k, s);
       else launch_col<T, -1>(ya, P[1], nl_y, gy, s);
     } else {
       ya.nvalid = P[1]; ya.nout = N[1];
       if (launch_coly<T, +1>(ya, P[1], N[2], s)) return;
-      if (ry.len.n && ty.sched == 0) rcol(dir, s);
+      if (ry.len.n && ty.sched == 0) rcol(dir, k, s);
       else launch_col<T, +1>(ya, P[1], nl_y, gy, s);
     }
   }
   // the convolution pass: Z (3D) or Y (2D) forward, tensor multiply, inverse
-  void pass_conv(hipStream_t s) {
+  void pass_conv(Cols k, hipStream_t s) {
     const T *K[6];
-    for (int c = 0; c < 6; c++) K[c] = kern.as<T>() + c * kcount;
+    for (int c = 0; c < 6; c++) K[c] = kern.as<T>() + c * kcount + k.x0;
     if (!is2d && zreg) {
       ConvZArgs<T> za{};
-      za.H = H; za.Py = P[1]; za.KHy = KHy; za.Hk = Hk; za.zstride = (long)P[1] * Hp; za.ystride = Hp;
-      za.nyq = H > 1 && (H - 1) % CONVZ_COLS == 0;
-      za.K = kern.as<T>();
-      for (int c = 0; c < 3; c++) za.buf[c] = spec[c].as<C2<T>>();
+      za.H = k.n; za.Py = P[1]; za.KHy = KHy; za.Hk = Hk; za.zstride = (long)P[1] * Hp; za.ystride = Hp;
+      za.nyq = k.n > 1 && (k.n - 1) % CONVZ_COLS == 0;
+      za.K = kern.as<T>() + k.x0;
+      for (int c = 0; c < 3; c++) za.buf[c] = spec[c].as<C2<T>>() + k.x0;
       launch_convz<T>(za, N[2], s);
       return;
     }
     if (rshort && tz.sched == 0) {
       RShortArgs<T> r{};
-      r.H = H; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk; r.zstride = (long)P[1] * Hp; r.ystride = Hp;
+      r.H = k.n; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk; r.zstride = (long)P[1] * Hp; r.ystride = Hp;
       for (int c = 0; c < 6; c++) r.K[c] = K[c];
-      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>();
+      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>() + k.x0;
       launch_rshort<T>(r, N[2], s);
       return;
     }
     if (rc.len.n && (is2d ? ty : tz).sched == 0) {
       RConvArgs<T> r{};
-      r.f = rc.len; r.lsh = log2i(rc.nl); r.H = H; r.nvalid = is2d ? N[1] : N[2];
+      r.f = rc.len; r.lsh = log2i(rc.nl); r.H = k.n; r.nvalid = is2d ? N[1] : N[2];
       r.estride = is2d ? Hp : (long)P[1] * Hp; r.pstride = is2d ? 0 : Hp;
       r.is2d = is2d; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk;
       for (int c = 0; c < 6; c++) r.K[c] = K[c];
-      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>();
+      for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>() + k.x0;
       launch_rconv<T>(r, rc.nt, s);
       return;
     }
     ConvArgs<T> ca{};
-    ca.f = is2d ? ty.len : tz.len; ca.B = B_conv; ca.fB.init(B_conv); ca.f3B.init(3 * B_conv); ca.H = H;
+    ca.f = is2d ? ty.len : tz.len; ca.B = B_conv; ca.fB.init(B_conv); ca.f3B.init(3 * B_conv); ca.H = k.n;
     ca.nvalid = is2d ? N[1] : N[2];
     ca.estride = is2d ? Hp : (long)P[1] * Hp; ca.pstride = is2d ? 0 : Hp;
     ca.is2d = is2d; ca.Py = P[1]; ca.Pz = is2d ? 1 : P[2]; ca.KHy = KHy; ca.Hk = Hk;
     for (int c = 0; c < 6; c++) ca.K[c] = K[c];
-    for (int c = 0; c < 3; c++) ca.buf[c] = spec[c].as<C2<T>>();
-    dim3 gc((H + B_conv - 1) / B_conv, is2d ? 1 : P[1] / 2 + 1);   // 3D: ky and Py-ky per work-group
+    for (int c = 0; c < 3; c++) ca.buf[c] = spec[c].as<C2<T>>() + k.x0;
+    dim3 gc((k.n + B_conv - 1) / B_conv, is2d ? 1 : P[1] / 2 + 1);   // 3D: ky and Py-ky per work-group
     launch_conv<T>(ca, is2d ? P[1] : P[2], B_conv, gc, s);
+  }
+  // Columns per run of the Y forward, Z and Y inverse passes.  A spectrum that
+  // exceeds the 256 MB last-level cache is taken in parts of at most 208 MB, so
+  // that a pass finds in the cache what the pass before it wrote (the cache
+  // moves 8.5 TB/s, HBM 5 to 6).  Convolution of 1024 x 1024 x 8 FP32 (403 MB)
+  // whole 767 us, in 2 parts 710; x 16 1538, 4 parts 1399; x 32 3010, 8 parts
+  // 2843; 400 x 400 x 40 804, 2 parts 783; 2000 x 1000 x 10 the same.  What fits
+  // gains nothing and fills its last round of work-groups worse (512 x 512 x 16,
+  // 202 MB: 277, 2 parts 293).  k_coly's lengths stay whole, one launch per pass:
+  // their wide tiles leave a gain at few of the sizes (512 x 512 x 32: 587, 2
+  // parts 562, 3 parts 595, 6 parts 692).  FP64 passes are bound by their
+  // arithmetic (512 x 512 x 32 1497, 4 parts 1535): never split.  Parts start on
+  // a 256-byte boundary of the rows.
+  int chunk_cols() const {
+    if (sizeof(T) != 4 || !ry.len.n || ty.sched != 0) return H;
+    const int parts = (int)ceil(3.0 * sizeof(C2<T>) * N[2] * P[1] * H / 208e6);
+    return parts > 1 ? std::max(32, (H / parts + 31) / 32 * 32) : H;
   }
   // X forward through Y inverse (3D) or the 2D Y pass: leaves the convolved
   // half spectrum (rows y < Ny) in spec[] for the X inverse.
   void spectral(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s) {
     pass_xfwd(mv, vol, Msa, Ms_mul, s);
-    if (!is2d) pass_y(-1, s);
-    pass_conv(s);
-    if (!is2d) pass_y(+1, s);
+    const int w = chunk_cols();
+    for (Cols k{0, 0}; k.x0 < H; k.x0 += k.n) {
+      k.n = H - k.x0 <= w + w / 4 ? H - k.x0 : w;
+      if (!is2d) pass_y(-1, k, s);
+      pass_conv(k, s);
+      if (!is2d) pass_y(+1, k, s);
+    }
   }
   void pass_xinv(void *const Bv[3], hipStream_t s) {
     XiArgs<T> a = xinv_args(nl_xi);
@@ -2204,7 +2226,7 @@ struct DemagPlan : DemagBase {
           for (int sc = 0; sc < FFT_NSCHED; sc++) {
             nl_y = nl;
             try { ty.schedule(sc); } catch (const Error &) { continue; }
-            const float t = timed([&] { pass_y(-1, s); pass_y(+1, s); });
+            const float t = timed([&] { const Cols k{0, H}; pass_y(-1, k, s); pass_y(+1, k, s); });
             if (t < best) { best = t; bn = nl; bs = sc; }
           }
         nl_y = bn;
@@ -2225,7 +2247,7 @@ struct DemagPlan : DemagBase {
           for (int sc = 0; sc < FFT_NSCHED; sc++) {
             B_conv = B;
             try { tc.schedule(sc); } catch (const Error &) { continue; }
-            const float t = timed([&] { pass_conv(s); });
+            const float t = timed([&] { pass_conv({0, H}, s); });
             if (t < best) { best = t; bb_ = B; bsc = sc; }
           }
         }
