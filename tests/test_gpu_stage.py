@@ -1,0 +1,72 @@
+"""Solver stages formed inside the X forward pass of the demag convolution
+(small grids): every solver's stages (2 to 6 sources, with and without
+normalisation), rows of one pair, remainders of a work-group, several z
+planes, a geometry, lengths with a compiled X pass and odd rows (which keep
+the separate stage kernel), and the largest component array that takes it.
+
+Against the FP64 oracle over 3 fixed steps.  dt gammaLL |B| is about 2e-3, so
+the convolution's 2e-6 adds 1e-8 and rounding m (6e-8 a stage, up to 6 stages
+a step) dominates FP32: 2e-6.  FP64: 1e-12 likewise."""
+import numpy as np
+import pytest
+
+from cases import random_unit
+from umagnus_amd.params import exchange_lut
+
+pytestmark = pytest.mark.gpu
+SOLVERS = (2, 3, 4, 5)   # Heun, RK23, RK4, RK45DP
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    from umagnus_amd import umhip
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    umhip.init(0)
+    return umhip
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float32, 2e-6), (np.float64, 1e-12)])
+@pytest.mark.parametrize("N,geom", [((2, 8, 1), False), ((30, 7, 1), True), ((10, 6, 5), False), ((64, 9, 2), True),
+                                    ((96, 5, 1), False), ((128, 32, 1), False), ((35, 6, 1), True)])
+def test_stages_match_oracle(gpu, oracle, N, geom, dtype, tol):
+    shape = (N[2], N[1], N[0])
+    for solver in SOLVERS:
+        print("stages", N, dtype.__name__, solver, flush=True)
+        out = []
+        for mod, dt in ((oracle, np.float64), (gpu, dtype)):
+            s = mod.Sim(N, (4e-9, 3e-9, 2e-9), dtype=dt)
+            s.set_scalar(mod.P_MSAT, 8e5)
+            s.set_scalar(mod.P_ALPHA, 0.1)
+            s.set_exchange_luts(exchange_lut(1.3e-11, dtype=dt), None)
+            if geom:
+                v = np.ones(shape, dt)
+                v.reshape(-1)[::5] = 0
+                v.reshape(-1)[1::7] = 0.5
+                s.set_geometry(v)
+            s.set_m(random_unit(shape, 3).astype(dt))
+            s.set_solver(solver)
+            s.set_solver_params(dt=1e-14, fixdt=1e-14)
+            s.steps(3)
+            out.append(np.asarray(s.get_m(), np.float64))
+        assert np.abs(out[0] - out[1]).max() <= tol, solver
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_largest_component_array(gpu, dtype):
+    """The largest component arrays up to 1 MiB take the path, the next ones do
+    not; m stays normalised on both."""
+    for rows, want in ((640, 12), (672, 0)) if dtype == np.float32 else ((320, 12), (336, 0)):
+        s = gpu.Sim((400, rows, 1), (4e-9, 3e-9, 2e-9), dtype=dtype)
+        s.set_scalar(gpu.P_MSAT, 8e5)
+        s.set_scalar(gpu.P_ALPHA, 0.1)
+        s.set_exchange_luts(exchange_lut(1.3e-11, dtype=dtype), None)
+        s.set_m(random_unit((1, rows, 400), 5).astype(dtype))
+        s.set_solver(5)
+        s.set_solver_params(dt=1e-14, fixdt=1e-14)
+        with gpu.KernelTrace() as tr:
+            s.steps(2)
+        fused = sum("k_rxstage" in k for k in tr.names)
+        assert fused == want, tr.names
+        m = np.asarray(s.get_m(), np.float64)
+        assert np.abs((m * m).sum(0) - 1).max() < 1e-6

@@ -25,6 +25,7 @@
 #include "batch.hpp"
 #include "demag_reg.hpp"
 #include "demag_x4.hpp"
+#include "stage_device.hpp"
 #include "fft_ct.hpp"
 #include "field.hpp"
 #include "sim.hpp"
@@ -1662,6 +1663,7 @@ struct DemagBase {
   virtual void kspec(int c, void *host) = 0;
   virtual bool exec_field(const void *const m[3], const void *vol, const void *Ms, double Ms_mul, const void *fa,
                           hipStream_t s) = 0;
+  virtual bool take_stage(const void *stage) = 0;
   virtual void schedule(int out[DEMAG_NKNOB]) const = 0;
   virtual void tune(hipStream_t s) = 0;
 };
@@ -1913,6 +1915,16 @@ struct DemagPlan : DemagBase {
     a.Nx = Nx; a.rows = Ny * Nz; a.fRy.init(Ny); a.Py = is2d ? Ny : P[1]; a.Hp = Hp; a.in_pitch = Nx;
     for (int c = 0; c < 3; c++) { a.src[c] = (const T *)mv[c]; a.out[c] = spec[c].as<C2<T>>(); }
     a.Ms = Par<T>{(const T *)Msa, (T)Ms_mul}; a.vol = (const T *)vol;
+    if (pending) {
+      RXStageArgs<T> r{rx_args(), *pending};
+      pending = nullptr;
+      r.x.in_pitch = Nx;
+      for (int c = 0; c < 3; c++) r.x.src[c] = (const T *)mv[c];
+      r.x.Ms = a.Ms; r.x.vol = a.vol;
+      r.x.pairs = even_pairs(r.x.src, a.Ms.arr, a.vol);
+      launch_rxstage<T>(r, rx.nt, s);
+      return;
+    }
     dim3 g((a.rows + nl_x - 1) / nl_x, 3);
     if (xodd) {
       a.f = tx2.len; a.fhalf.init(H);
@@ -1930,6 +1942,26 @@ struct DemagPlan : DemagBase {
         launch_xfwd<T>(a, P[0] / 2, nl_x, g, s);
       }
     }
+  }
+  // A solver stage as part of the next X forward pass: the register pass forms
+  // its rows of m, stores them and transforms them, which saves a launch whose
+  // 4 to 6 us are nearly all start and drain.  Each component's work-group sums
+  // all three components, so the sources are read three times: only while a
+  // component array is at most 1 MiB.  RK45DP, 8 replayed steps, apart -> in
+  // one, us: 64 x 64 FP64 1285 -> 1179, 256 x 256 FP64 1970 -> 1860; 250 x 250
+  // FP32 (9 steps) 2229 -> 2130; 160 x 160 x 10 FP32 (RK4) 990 -> 942.  Above:
+  // 70^3 FP64 1694 -> 1762, 1000 x 1000 FP32 (Heun) 1156 -> 1162.  Only lengths
+  // whose X forward is the register pass anyway, so m does not depend on which
+  // entry point formed it beyond the stage's own rounding.  false: not taken.
+  static constexpr size_t STAGE_BYTES = 1 << 20;
+  const StageArgs<T> *pending = nullptr;
+  bool take_stage(const void *sv) override {
+    pending = nullptr;
+    if (!sv) return false;
+    const StageArgs<T> &a = *(const StageArgs<T> *)sv;
+    if (!fused_field || !rx.len.n || tx.sched != 0 || sizeof(T) * a.N > STAGE_BYTES || !stage_pair_ok(a, N[0])) return false;
+    pending = &a;
+    return true;
   }
   // pairwise access to real rows: even Nx and every array aligned to two values
   template <typename Q>
@@ -2452,6 +2484,7 @@ void demag_exec(DemagBase *d, void *const B[3], const void *const m[3], const vo
                 double Ms_mul, hipStream_t s) {
   d->exec(B, m, vol, Ms, Ms_mul, s);
 }
+bool demag_take_stage(DemagBase *d, const void *stage) { return d->take_stage(stage); }
 bool demag_exec_field(DemagBase *d, const void *const m[3], const void *vol, const void *Ms, double Ms_mul,
                       const void *fa, hipStream_t s) {
   return d->exec_field(m, vol, Ms, Ms_mul, fa, s);

@@ -13,6 +13,7 @@
 
 #include "batch.hpp"
 #include "fft.hpp"
+#include "vec.hpp"
 
 namespace um {
 
@@ -76,6 +77,11 @@ struct RXArgs {
   C2<T> *spec[3];
   T *dst[3];              // inverse: real rows of Nx
 };
+template <typename T>
+struct RXStageArgs {
+  RXArgs<T> x;
+  StageArgs<T> st;        // the solver stage that forms the input rows
+};
 // column pass along y
 template <typename T>
 struct RColArgs {
@@ -107,6 +113,7 @@ struct RShortArgs {
 
 template <typename T> void launch_rxfwd(const RXArgs<T> &a, int nt, hipStream_t s);
 template <typename T> void launch_rxinv(const RXArgs<T> &a, int nt, hipStream_t s);
+template <typename T> void launch_rxstage(const RXStageArgs<T> &a, int nt, hipStream_t s);
 template <typename T> void launch_rcol(const RColArgs<T> &a, int dir, int planes, int nt, hipStream_t s);
 template <typename T> void launch_rconv(const RConvArgs<T> &a, int nt, hipStream_t s);
 template <typename T> bool short_ok(int Nz, int Pz);

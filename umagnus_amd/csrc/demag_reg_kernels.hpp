@@ -2,6 +2,7 @@
 #pragma once
 #include "demag_reg.hpp"
 #include "fft_device.hpp"
+#include "stage_device.hpp"
 
 namespace um {
 
@@ -220,6 +221,24 @@ struct BRXfwd {
 };
 template <typename T>
 __global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 1) void k_rxfwd(RXArgs<T> a) { BRXfwd<T>::run(a, hw_bid(), hw_grid()); }
+
+// X forward of rows that a solver stage forms first: the work-group stores its
+// rows of one component, then transforms what it stored.
+template <typename T>
+struct BRXStage {
+  using Args = RXStageArgs<T>;
+  static constexpr int NT = 512, MINB = sizeof(T) == 4 ? 4 : 1;
+  static __device__ __forceinline__ void run(const RXStageArgs<T> &as, uint3 blockIdx, uint3 gridDim) {
+    const RXArgs<T> &a = as.x;
+    const int row0 = blockIdx.x * a.nl, pairs = min(a.nl, a.rows - row0) * (a.Nx / 2);
+    if (!(as.st.skip && *as.st.skip))
+      for (int g = threadIdx.x; g < pairs; g += blockDim.x) stage_pair(as.st, blockIdx.y, (long)row0 * a.Nx + 2 * g);
+    __syncthreads();
+    BRXfwd<T>::run(a, blockIdx, gridDim);
+  }
+};
+template <typename T>
+__global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 1) void k_rxstage(RXStageArgs<T> a) { BRXStage<T>::run(a, hw_bid(), hw_grid()); }
 
 // ---- X inverse -----------------------------------------------------------------
 // One LDS round trip less than the forward pass: the last stage's lanes hold
@@ -618,6 +637,13 @@ void launch_rxinv(const RXArgs<T> &a, int nt, hipStream_t s) {
   UM_HIP(hipGetLastError());
 }
 template <typename T>
+void launch_rxstage(const RXStageArgs<T> &a, int nt, hipStream_t s) {
+  const size_t lds = sizeof(C2<T>) * (size_t)a.x.nl * a.x.f.line();
+  reg_lds(k_rxstage<T>, lds);
+  launch_b<BRXStage<T>>(k_rxstage<T>, dim3((a.x.rows + a.x.nl - 1) / a.x.nl, 3), dim3(nt), lds, s, a);
+  UM_HIP(hipGetLastError());
+}
+template <typename T>
 void launch_rcol(const RColArgs<T> &a, int dir, int planes, int nt, hipStream_t s) {
   const size_t lds = sizeof(C2<T>) * ((size_t)a.f.line() << a.lsh);
   const dim3 grid((a.H + (1 << a.lsh) - 1) >> a.lsh, planes, 3);
@@ -688,6 +714,7 @@ void RegTab<T>::bind(const C2<T> *dev) {
 #define UM_REG_INSTANTIATE(T)                                              \
   template void launch_rxfwd<T>(const RXArgs<T> &, int, hipStream_t);      \
   template void launch_rxinv<T>(const RXArgs<T> &, int, hipStream_t);      \
+  template void launch_rxstage<T>(const RXStageArgs<T> &, int, hipStream_t); \
   template void launch_rcol<T>(const RColArgs<T> &, int, int, int, hipStream_t); \
   template void launch_rconv<T>(const RConvArgs<T> &, int, hipStream_t);   \
   template void launch_rshort<T>(const RShortArgs<T> &, int, hipStream_t); \

@@ -640,6 +640,26 @@ struct Sim : SimBase {
   // m_out = normalize(sum fac_j src_j)
   void stage(T *dst, int ns, const T *const *src, const T *fac, bool norm, bool group3 = false,
              T *nrm = nullptr) {
+    launch_stage(stage_args(dst, ns, src, fac, norm, group3, nrm), st);
+  }
+  // a stage into m and the torque of the result: the demag plan may form m in
+  // its X forward pass
+  void stage_torque(int ns, const T *const *src, const T *fac, bool norm, bool group3, T *kout) {
+    const StageArgs<T> a = stage_args(m, ns, src, fac, norm, group3, nullptr);
+    bool taken = false;
+    if (enable_demag && !has_nodemag) {
+      ensure_demag();
+      taken = demag_take_stage(demag, &a);
+    }
+    if (!taken) launch_stage(a, st);
+    try {
+      torque_fn(kout);
+    } catch (...) {
+      if (taken) demag_take_stage(demag, nullptr);   // the plan keeps no pointer to a
+      throw;
+    }
+  }
+  StageArgs<T> stage_args(T *dst, int ns, const T *const *src, const T *fac, bool norm, bool group3, T *nrm) {
     StageArgs<T> a{};
     a.nrm = nrm;
     a.nsrc = ns;
@@ -659,7 +679,7 @@ struct Sim : SimBase {
       a.gam = gammaLL;
       a.skip = &d->done;
     }
-    launch_stage(a, st);
+    return a;
   }
   // device statistics of a captured step (count: its last statistics launch)
   void step_stats(double h, int mode, bool count) {
@@ -703,38 +723,33 @@ struct Sim : SimBase {
       const T *s[] = {m0, k1};
       const T f[] = {T(1), T(1. / 5.) * h};
       Time = t0 + (1. / 5.) * dt;
-      stage(m, 2, s, f, true);
-      torque_fn(k2);
+      stage_torque(2, s, f, true, false, k2);
     }
     {
       const T *s[] = {m0, k1, k2};
       const T f[] = {T(1), T(3. / 40.) * h, T(9. / 40.) * h};
       Time = t0 + (3. / 10.) * dt;
-      stage(m, 3, s, f, true, true);
-      torque_fn(k3);
+      stage_torque(3, s, f, true, true, k3);
     }
     {
       const T *s[] = {m0, k1, k2, k3};
       const T f[] = {T(1), T(44. / 45.) * h, T(-56. / 15.) * h, T(32. / 9.) * h};
       Time = t0 + (4. / 5.) * dt;
-      stage(m, 4, s, f, true);
-      torque_fn(k4);
+      stage_torque(4, s, f, true, false, k4);
     }
     {
       const T *s[] = {m0, k1, k2, k3, k4};
       const T f[] = {T(1), T(19372. / 6561.) * h, T(-25360. / 2187.) * h, T(64448. / 6561.) * h,
                      T(-212. / 729.) * h};
       Time = t0 + (8. / 9.) * dt;
-      stage(m, 5, s, f, true);
-      torque_fn(k5);
+      stage_torque(5, s, f, true, false, k5);
     }
     {
       const T *s[] = {m0, k1, k2, k3, k4, k5};
       const T f[] = {T(1), T(9017. / 3168.) * h, T(-355. / 33.) * h, T(46732. / 5247.) * h,
                      T(49. / 176.) * h, T(-5103. / 18656.) * h};
       Time = t0 + dt;
-      stage(m, 6, s, f, true);
-      torque_fn(k6);
+      stage_torque(6, s, f, true, false, k6);
     }
     T *k7 = k2;
     {
@@ -742,8 +757,7 @@ struct Sim : SimBase {
       const T f[] = {T(1), T(35. / 384.) * h, T(500. / 1113.) * h, T(125. / 192.) * h,
                      T(-2187. / 6784.) * h, T(11. / 84.) * h};
       Time = t0 + dt;
-      stage(m, 6, s, f, true);
-      torque_fn(k7);
+      stage_torque(6, s, f, true, false, k7);
     }
     const T e[6] = {T(35. / 384. - 5179. / 57600.), T(500. / 1113. - 7571. / 16695.),
                     T(125. / 192. - 393. / 640.), T(-2187. / 6784. - -92097. / 339200.),
@@ -805,15 +819,13 @@ struct Sim : SimBase {
       const T *s[] = {m0, k1};
       const T f[] = {T(1), T(1. / 2.) * h};
       Time = t0 + (1. / 2.) * dt;
-      stage(m, 2, s, f, true);
-      torque_fn(k2);
+      stage_torque(2, s, f, true, false, k2);
     }
     {
       const T *s[] = {m0, k2};
       const T f[] = {T(1), T(3. / 4.) * h};
       Time = t0 + (3. / 4.) * dt;
-      stage(m, 2, s, f, true);
-      torque_fn(k3);
+      stage_torque(2, s, f, true, false, k3);
     }
     {
       const T *s[] = {m0, k1, k2, k3};
@@ -869,13 +881,12 @@ struct Sim : SimBase {
     UM_REQUIRE(h > 0, UM_ESTATE, "dt must be positive");
     torque_fn(dy0);
     std::swap(m, m0);
+    Time += dt;
     {
       const T *s[] = {m0, dy0};
       const T f[] = {T(1), h};
-      stage(m, 2, s, f, false);   // stage 1 is not normalised (heun.go:32)
+      stage_torque(2, s, f, false, false, dy);   // stage 1 is not normalised (heun.go:32)
     }
-    Time += dt;
-    torque_fn(dy);
     double r[3];
     const T *src[2] = {dy0, dy};
     err_reduce(1, src, 2, nullptr, r);
@@ -910,13 +921,10 @@ struct Sim : SimBase {
     torque_fn(k1);
     std::swap(m, m0);
     Time = t0 + (1. / 2.) * dt;
-    { const T *s[] = {m0, k1}; const T f[] = {T(1), T(1. / 2.) * h}; stage(m, 2, s, f, true); }
-    torque_fn(k2);
-    { const T *s[] = {m0, k2}; const T f[] = {T(1), T(1. / 2.) * h}; stage(m, 2, s, f, true); }
-    torque_fn(k3);
+    { const T *s[] = {m0, k1}; const T f[] = {T(1), T(1. / 2.) * h}; stage_torque(2, s, f, true, false, k2); }
+    { const T *s[] = {m0, k2}; const T f[] = {T(1), T(1. / 2.) * h}; stage_torque(2, s, f, true, false, k3); }
     Time = t0 + dt;
-    { const T *s[] = {m0, k3}; const T f[] = {T(1), T(1.) * h}; stage(m, 2, s, f, true); }
-    torque_fn(k4);
+    { const T *s[] = {m0, k3}; const T f[] = {T(1), T(1.) * h}; stage_torque(2, s, f, true, false, k4); }
     double r[3];
     const T *src[2] = {k1, k4};
     err_reduce(1, src, 2, nullptr, r);

@@ -35,6 +35,11 @@ void demag_exec(DemagBase *d, void *const B[3], const void *const m[3], const vo
 // plan's precision (bd unused).  false when the plan has no fused path.
 bool demag_exec_field(DemagBase *d, const void *const m[3], const void *vol, const void *Ms, double Ms_mul,
                       const void *fa, hipStream_t s);
+// Hands the plan a solver stage (StageArgs of its precision, alive until then)
+// whose result is the m of the convolution enqueued next: its X forward pass
+// forms and stores m itself.  false when the plan does not take it (the caller
+// launches the stage).  nullptr: takes back one not yet used.
+bool demag_take_stage(DemagBase *d, const void *stage);
 void demag_destroy(DemagBase *d);
 void demag_kspec(DemagBase *d, int c, void *host);
 void demag_info(DemagBase *d, int P[3], int *prec);
