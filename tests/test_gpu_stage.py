@@ -70,3 +70,45 @@ def test_largest_component_array(gpu, dtype):
         assert fused == want, tr.names
         m = np.asarray(s.get_m(), np.float64)
         assert np.abs((m * m).sum(0) - 1).max() < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("solver", SOLVERS)
+def test_time_functions_see_the_stage(gpu, monkeypatch, solver, dtype):
+    """A time function, of a parameter or of a field term, that reads m finds
+    every stage's m in it: what it reads, and a trajectory fed back from it, are
+    those of a handle whose stages are always kernels of their own."""
+    N = (30, 14, 2)
+    shape = (N[2], N[1], N[0])
+    for term in (False, True):
+        print("time function", solver, dtype.__name__, term, flush=True)
+        runs = []
+        for fused in ("1", "0"):
+            monkeypatch.setenv("UMHIP_FUSED_FIELD", fused)
+            s = gpu.Sim(N, (4e-9, 3e-9, 2e-9), dtype=dtype)
+            s.set_scalar(gpu.P_MSAT, 8e5)
+            s.set_scalar(gpu.P_ALPHA, 0.1)
+            s.set_exchange_luts(exchange_lut(1.3e-11, dtype=dtype), None)
+            s.set_m(random_unit(shape, 9).astype(dtype))
+            s.set_solver(solver)
+            s.set_solver_params(dt=1e-13, fixdt=1e-13)
+            seen = []
+
+            def feedback(t):
+                seen.append(np.array(s.get_m()))
+                return 0.05 * s.average_m()[0]
+
+            if term:
+                s.add_field_term(s.FIELD_TERM_CUSTOM, random_unit(shape, 4).astype(dtype), fn=feedback)
+            else:
+                s.set_time_function(gpu.P_BEXT, lambda t: (feedback(t), 0.0, 0.0), 3)
+            s.steps(3)
+            runs.append((seen, np.array(s.get_m())))
+        (seen, m), (want, mw) = runs
+        assert len(seen) == len(want) >= 6
+        # FixDt of 1e-13 turns m by 1e-2 a step: no stage repeats the one before
+        for i in range(1, len(want)):
+            assert not np.array_equal(want[i], want[i - 1]), i
+        for i, (a, b) in enumerate(zip(seen, want)):
+            assert np.array_equal(a, b), (i, np.abs(a.astype(float) - b).max())
+        assert np.array_equal(m, mw)

@@ -643,11 +643,13 @@ struct Sim : SimBase {
     launch_stage(stage_args(dst, ns, src, fac, norm, group3, nrm), st);
   }
   // a stage into m and the torque of the result: the demag plan may form m in
-  // its X forward pass
+  // its X forward pass.  Not with time functions: torque_fn calls them before
+  // the convolution is enqueued, and they may read m (get_m, average_m,
+  // m_device), which must then hold the stage.
   void stage_torque(int ns, const T *const *src, const T *fac, bool norm, bool group3, T *kout) {
     const StageArgs<T> a = stage_args(m, ns, src, fac, norm, group3, nullptr);
     bool taken = false;
-    if (enable_demag && !has_nodemag) {
+    if (enable_demag && !has_nodemag && !any_tfn && !xterm_tfn) {
       ensure_demag();
       taken = demag_take_stage(demag, &a);
     }
