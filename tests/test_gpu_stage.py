@@ -112,3 +112,45 @@ def test_time_functions_see_the_stage(gpu, monkeypatch, solver, dtype):
         for i, (a, b) in enumerate(zip(seen, want)):
             assert np.array_equal(a, b), (i, np.abs(a.astype(float) - b).max())
         assert np.array_equal(m, mw)
+
+
+# rows of one pair, remainders of a work-group, periodic axes (half and odd
+# lengths), several planes, the largest component array that takes the path
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("N,pbc", [((2, 8, 1), (0, 0, 0)), ((30, 7, 1), (0, 0, 0)), ((30, 20, 3), (2, 0, 0)),
+                                   ((42, 10, 1), (0, 1, 0)), ((20, 12, 5), (1, 1, 1)), ((250, 50, 1), (0, 0, 0)),
+                                   ((160, 16, 10), (0, 0, 0)), ((400, 320, 1), (0, 0, 0))])
+def test_same_bits_as_separate_stages(gpu, monkeypatch, N, pbc, dtype):
+    """m after fixed and after device-controlled adaptive steps does not depend
+    on which kernel forms the stages."""
+    shape = (N[2], N[1], N[0])
+    for solver, geom in ((2, False), (3, True), (4, False), (5, True), (5, False)):
+        print("same bits", N, pbc, dtype.__name__, solver, geom, flush=True)
+        out, fused = [], []
+        for env in ("1", "0"):
+            monkeypatch.setenv("UMHIP_FUSED_FIELD", env)
+            s = gpu.Sim(N, (4e-9, 3e-9, 2e-9), pbc=pbc, dtype=dtype)
+            s.set_scalar(gpu.P_MSAT, 8e5)
+            s.set_scalar(gpu.P_ALPHA, 0.1)
+            s.set_exchange_luts(exchange_lut(1.3e-11, dtype=dtype), None)
+            if geom:
+                v = np.ones(shape, dtype)
+                v.reshape(-1)[::5] = 0
+                v.reshape(-1)[1::7] = 0.5
+                s.set_geometry(v)
+            s.set_m(random_unit(shape, 6).astype(dtype))
+            s.set_solver(solver)
+            s.set_solver_params(dt=1e-13, fixdt=1e-13)
+            with gpu.KernelTrace() as tr:
+                s.steps(3)
+            fused.append(sum("k_rxstage" in k for k in tr.names))
+            m = [np.array(s.get_m())]
+            if solver == 5:
+                s.set_graph(1)
+                s.set_solver_params(dt=1e-14)
+                s.run(3e-13)
+                m.append(np.array(s.get_m()))
+            out.append(m)
+        assert fused[0] > 0 and fused[1] == 0, fused
+        for a, b in zip(*out):
+            assert np.array_equal(a, b), np.abs(a.astype(float) - b).max()

@@ -1951,8 +1951,8 @@ struct DemagPlan : DemagBase {
   // one, us: 64 x 64 FP64 1285 -> 1179, 256 x 256 FP64 1970 -> 1860; 250 x 250
   // FP32 (9 steps) 2229 -> 2130; 160 x 160 x 10 FP32 (RK4) 990 -> 942.  Above:
   // 70^3 FP64 1694 -> 1762, 1000 x 1000 FP32 (Heun) 1156 -> 1162.  Only lengths
-  // whose X forward is the register pass anyway, so m does not depend on which
-  // entry point formed it beyond the stage's own rounding.  false: not taken.
+  // whose X forward is the register pass anyway, so m has the same bits
+  // whichever kernel formed it.  false: not taken.
   static constexpr size_t STAGE_BYTES = 1 << 20;
   const StageArgs<T> *pending = nullptr;
   bool take_stage(const void *sv) override {

@@ -8,9 +8,13 @@ namespace um {
 
 // Component c of the stage at cells i and i + 1.  All
 // three components are summed, since the norm needs them; up to 18 loads are
-// in flight.
+// in flight.  Every product and fused multiply-add is written out: they are
+// those of k_stage (vec.hip), which runs the stages of the same grids where
+// this form does not apply (time functions, the tape), so m has the same bits
+// whichever kernel forms it.
 template <typename T, int NS>
 __device__ __forceinline__ void stage_pair_n(const StageArgs<T> &s, int c, long i) {
+#pragma clang fp contract(off)
   const T h = s.dev_dt ? (T)(s.dev_dt[0] * s.gam) : T(1);
   C2<T> x[3][NS], vv{T(1), T(1)};
 #pragma unroll
@@ -25,20 +29,22 @@ __device__ __forceinline__ void stage_pair_n(const StageArgs<T> &s, int c, long 
   for (int w = 0; w < 2; w++) {
 #pragma unroll
     for (int e = 0; e < 3; e++) {
-      auto at = [&](int k) { return w ? x[e][k].y : x[e][k].x; };
-      T acc = f[0] * at(0);
+      T u[NS];
+#pragma unroll
+      for (int k = 0; k < NS; k++) u[k] = w ? x[e][k].y : x[e][k].x;
+      T acc = f[0] * u[0];
       if (NS == 3 && s.group3) {
-        acc = acc + (f[1] * at(1) + f[2] * at(2));
+        acc = acc + fma(f[1], u[1], f[2] * u[2]);
       } else {
 #pragma unroll
-        for (int k = 1; k < NS; k++) acc = acc + f[k] * at(k);
+        for (int k = 1; k < NS; k++) acc = fma(f[k], u[k], acc);
       }
       r[w][e] = acc;
     }
     if (s.normalize) {   // normalize2.cl:8-23
       const T v = w ? vv.y : vv.x;
       const T X = v * r[w][0], Y = v * r[w][1], Z = v * r[w][2];
-      const T l = sqrt(X * X + Y * Y + Z * Z);
+      const T l = sqrt(fma(Z, Z, fma(X, X, Y * Y)));
       const T inv = (l != T(0)) ? T(1) / l : T(0);
       r[w][0] = v == T(0) ? T(0) : X * inv;
       r[w][1] = v == T(0) ? T(0) : Y * inv;
