@@ -347,7 +347,8 @@ int um_sim_set_nodemag_lut(void *sim, const void *lut);
  * ctx) writes the parameter's ncomp (1 or 3) uniform multipliers at stage time
  * t before every effective-field evaluation; a per-cell array set with
  * um_sim_set_scalar/_vector is scaled by them.  fn = NULL removes it.  Steps
- * with a time function are not graph-replayed. */
+ * with a time function are not graph-replayed.  fn may read the handle (m is
+ * that of the stage) and change its parameters and flags. */
 typedef void (*um_time_fn)(double t, double *values, void *ctx);
 int um_sim_set_time_function(void *sim, int param, int ncomp, um_time_fn fn, void *ctx);
 /* Extra per-cell field and torque terms, each a host array per component

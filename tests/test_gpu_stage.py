@@ -154,3 +154,36 @@ def test_same_bits_as_separate_stages(gpu, monkeypatch, N, pbc, dtype):
         assert fused[0] > 0 and fused[1] == 0, fused
         for a, b in zip(*out):
             assert np.array_equal(a, b), np.abs(a.astype(float) - b).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_time_function_switches_demag(gpu, monkeypatch, dtype):
+    """A time function that switches the demag field off and on between stages:
+    every stage is formed all the same."""
+    N, shape = (30, 14, 2), (2, 14, 30)
+    out = []
+    for fused in ("1", "0"):
+        monkeypatch.setenv("UMHIP_FUSED_FIELD", fused)
+        s = gpu.Sim(N, (4e-9, 3e-9, 2e-9), dtype=dtype)
+        s.set_scalar(gpu.P_MSAT, 8e5)
+        s.set_scalar(gpu.P_ALPHA, 0.1)
+        s.set_exchange_luts(exchange_lut(1.3e-11, dtype=dtype), None)
+        s.set_m(random_unit(shape, 2).astype(dtype))
+        s.set_solver(5)
+        s.set_solver_params(dt=1e-13, fixdt=1e-13)
+        calls = [0]
+
+        def switch(t):
+            calls[0] += 1
+            s.set_flags(int(calls[0] % 3 != 0))
+            return (0.01, 0.0, 0.0)
+
+        s.set_time_function(gpu.P_BEXT, switch, 3)
+        print("switch", dtype.__name__, fused, flush=True)
+        s.steps(4)
+        s.set_time_function(gpu.P_BEXT, None, 3)
+        s.set_flags(1)
+        s.steps(2)
+        out.append(np.array(s.get_m()))
+    assert np.array_equal(*out)
+    assert np.abs((out[0].astype(float) ** 2).sum(0) - 1).max() < 1e-6

@@ -1659,11 +1659,11 @@ struct DemagBase {
   int prec = UM_F32;
   int N[3], P[3];
   virtual void exec(void *const B[3], const void *const m[3], const void *vol, const void *Ms,
-                    double Ms_mul, hipStream_t s) = 0;
+                    double Ms_mul, hipStream_t s, const void *stage) = 0;
   virtual void kspec(int c, void *host) = 0;
   virtual bool exec_field(const void *const m[3], const void *vol, const void *Ms, double Ms_mul, const void *fa,
                           hipStream_t s) = 0;
-  virtual bool take_stage(const void *stage) = 0;
+  virtual bool takes_stage(const void *stage) const = 0;
   virtual void schedule(int out[DEMAG_NKNOB]) const = 0;
   virtual void tune(hipStream_t s) = 0;
 };
@@ -1908,16 +1908,16 @@ struct DemagPlan : DemagBase {
 
   // X-fwd through Y-inv (3D) or the 2D Y pass: leaves the convolved half
   // spectrum (rows y < Ny) in spec[] for the X inverse.
-  void pass_xfwd(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s) {
+  void pass_xfwd(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s,
+                 const StageArgs<T> *stage = nullptr) {
     const int Nx = N[0], Ny = N[1], Nz = N[2];
     XArgs<T> a{};
     a.f = tx.len; a.tw2 = (const C2<T> *)tx2.buf.p; a.mode = 0; a.nl = nl_x; a.fhalf.init(P[0] / 4 + 1);
     a.Nx = Nx; a.rows = Ny * Nz; a.fRy.init(Ny); a.Py = is2d ? Ny : P[1]; a.Hp = Hp; a.in_pitch = Nx;
     for (int c = 0; c < 3; c++) { a.src[c] = (const T *)mv[c]; a.out[c] = spec[c].as<C2<T>>(); }
     a.Ms = Par<T>{(const T *)Msa, (T)Ms_mul}; a.vol = (const T *)vol;
-    if (pending) {
-      RXStageArgs<T> r{rx_args(), *pending};
-      pending = nullptr;
+    if (stage) {
+      RXStageArgs<T> r{rx_args(), *stage};
       r.x.in_pitch = Nx;
       for (int c = 0; c < 3; c++) r.x.src[c] = (const T *)mv[c];
       r.x.Ms = a.Ms; r.x.vol = a.vol;
@@ -1943,7 +1943,7 @@ struct DemagPlan : DemagBase {
       }
     }
   }
-  // A solver stage as part of the next X forward pass: the register pass forms
+  // A solver stage as part of the X forward pass (exec's stage): the register pass forms
   // its rows of m, stores them and transforms them, which saves a launch whose
   // 4 to 6 us are nearly all start and drain.  Each component's work-group sums
   // all three components, so the sources are read three times: only while a
@@ -1952,16 +1952,11 @@ struct DemagPlan : DemagBase {
   // FP32 (9 steps) 2229 -> 2130; 160 x 160 x 10 FP32 (RK4) 990 -> 942.  Above:
   // 70^3 FP64 1694 -> 1762, 1000 x 1000 FP32 (Heun) 1156 -> 1162.  Only lengths
   // whose X forward is the register pass anyway, so m has the same bits
-  // whichever kernel formed it.  false: not taken.
+  // whichever kernel formed it.
   static constexpr size_t STAGE_BYTES = 1 << 20;
-  const StageArgs<T> *pending = nullptr;
-  bool take_stage(const void *sv) override {
-    pending = nullptr;
-    if (!sv) return false;
+  bool takes_stage(const void *sv) const override {
     const StageArgs<T> &a = *(const StageArgs<T> *)sv;
-    if (!fused_field || !rx.len.n || tx.sched != 0 || sizeof(T) * a.N > STAGE_BYTES || !stage_pair_ok(a, N[0])) return false;
-    pending = &a;
-    return true;
+    return fused_field && rx.len.n && tx.sched == 0 && sizeof(T) * a.N <= STAGE_BYTES && stage_pair_ok(a, N[0]);
   }
   // pairwise access to real rows: even Nx and every array aligned to two values
   template <typename Q>
@@ -2062,8 +2057,9 @@ struct DemagPlan : DemagBase {
   }
   // X forward through Y inverse (3D) or the 2D Y pass: leaves the convolved
   // half spectrum (rows y < Ny) in spec[] for the X inverse.
-  void spectral(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s) {
-    pass_xfwd(mv, vol, Msa, Ms_mul, s);
+  void spectral(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s,
+                const StageArgs<T> *stage = nullptr) {
+    pass_xfwd(mv, vol, Msa, Ms_mul, s, stage);
     const int w = chunk_cols();
     for (Cols k{0, 0}; k.x0 < H; k.x0 += k.n) {
       k.n = H - k.x0 <= w + w / 4 ? H - k.x0 : w;
@@ -2101,8 +2097,8 @@ struct DemagPlan : DemagBase {
   }
 
   void exec(void *const Bv[3], const void *const mv[3], const void *vol, const void *Msa,
-            double Ms_mul, hipStream_t s) override {
-    spectral(mv, vol, Msa, Ms_mul, s);
+            double Ms_mul, hipStream_t s, const void *stage) override {
+    spectral(mv, vol, Msa, Ms_mul, s, (const StageArgs<T> *)stage);
     pass_xinv(Bv, s);
   }
 
@@ -2481,10 +2477,10 @@ void demag_kernel_mirror(const int P[3], double *const K[6], hipStream_t s) {
 }
 
 void demag_exec(DemagBase *d, void *const B[3], const void *const m[3], const void *vol, const void *Ms,
-                double Ms_mul, hipStream_t s) {
-  d->exec(B, m, vol, Ms, Ms_mul, s);
+                double Ms_mul, hipStream_t s, const void *stage) {
+  d->exec(B, m, vol, Ms, Ms_mul, s, stage);
 }
-bool demag_take_stage(DemagBase *d, const void *stage) { return d->take_stage(stage); }
+bool demag_takes_stage(DemagBase *d, const void *stage) { return d->takes_stage(stage); }
 bool demag_exec_field(DemagBase *d, const void *const m[3], const void *vol, const void *Ms, double Ms_mul,
                       const void *fa, hipStream_t s) {
   return d->exec_field(m, vol, Ms, Ms_mul, fa, s);

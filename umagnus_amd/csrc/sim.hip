@@ -502,7 +502,7 @@ struct Sim : SimBase {
   }
   // B_demag into bd (SetDemagField, engine/demag.go:42-65); with NoDemagSpins
   // the flagged cells neither generate nor receive the field (:67-98)
-  void compute_demag(const T *mm) {
+  void compute_demag(const T *mm, const StageArgs<T> *stg = nullptr) {
     if (!enable_demag) return;
     ensure_demag();
     void *B[3] = {bd, bd + n, bd + 2 * n};
@@ -512,7 +512,7 @@ struct Sim : SimBase {
       nodemag_input();
       v = ndvol.p;
     }
-    demag_exec(demag, B, mv, v, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul, st);
+    demag_exec(demag, B, mv, v, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul, st, stg);
     if (has_nodemag)
       for (int c = 0; c < 3; c++)
         zeromask<T>(bd + c * n, nodemagLUT.p, has_regions ? (const uint8_t *)regions.p : nullptr, n, st);
@@ -539,7 +539,8 @@ struct Sim : SimBase {
     }
     evused = 0;
   }
-  void torque_fn(T *dst) {
+  // stg: the stage that forms m, where the convolution takes it (stage_torque)
+  void torque_fn(T *dst, const StageArgs<T> *stg = nullptr) {
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
     if (profiling) {
       e0 = next_event();
@@ -554,13 +555,14 @@ struct Sim : SimBase {
       a.beff[c] = nullptr;
     }
     bool fused = false;
+    UM_REQUIRE(!stg || enable_demag, UM_ESTATE, "a solver stage without its convolution");
     if (enable_demag) {
       // one pipeline: B_demag stays on chip (the field share is timed with the demag)
       ensure_demag();
       const void *mv[3] = {m, m + n, m + 2 * n};
-      if (!has_nodemag)
+      if (!has_nodemag && !stg)
         fused = demag_exec_field(demag, mv, vol.p, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul, &a, st);
-      if (!fused) compute_demag(m);
+      if (!fused) compute_demag(m, stg);
     }
     if (profiling) UM_HIP(hipEventRecord(e1, st));
     if (!fused) launch_field_torque(a, st);
@@ -651,15 +653,10 @@ struct Sim : SimBase {
     bool taken = false;
     if (enable_demag && !has_nodemag && !any_tfn && !xterm_tfn) {
       ensure_demag();
-      taken = demag_take_stage(demag, &a);
+      taken = demag_takes_stage(demag, &a);
     }
     if (!taken) launch_stage(a, st);
-    try {
-      torque_fn(kout);
-    } catch (...) {
-      if (taken) demag_take_stage(demag, nullptr);   // the plan keeps no pointer to a
-      throw;
-    }
+    torque_fn(kout, taken ? &a : nullptr);
   }
   StageArgs<T> stage_args(T *dst, int ns, const T *const *src, const T *fac, bool norm, bool group3, T *nrm) {
     StageArgs<T> a{};

@@ -29,17 +29,16 @@ void kernel_ranges(const int P[3], const int pbc[3], int r1[3], int r2[3]);
 // first offset >= r1 that wraps onto w (0 <= w < P, r1 <= 0); the periodic
 // images of w are image_first, +P, +2P, ... up to r2
 __host__ __device__ __forceinline__ int image_first(int w, int P, int r1) { return w - P * ((w - r1) / P); }
+// stage (nullptr: none): a solver stage (StageArgs of the plan's precision)
+// that forms m, for which demag_takes_stage holds; the X forward pass forms
+// and stores m itself.
 void demag_exec(DemagBase *d, void *const B[3], const void *const m[3], const void *vol, const void *Ms,
-                double Ms_mul, hipStream_t s);
+                double Ms_mul, hipStream_t s, const void *stage = nullptr);
+bool demag_takes_stage(DemagBase *d, const void *stage);
 // Demag + effective field + torque in one pipeline; fa: FieldArgs of the
 // plan's precision (bd unused).  false when the plan has no fused path.
 bool demag_exec_field(DemagBase *d, const void *const m[3], const void *vol, const void *Ms, double Ms_mul,
                       const void *fa, hipStream_t s);
-// Hands the plan a solver stage (StageArgs of its precision, alive until then)
-// whose result is the m of the convolution enqueued next: its X forward pass
-// forms and stores m itself.  false when the plan does not take it (the caller
-// launches the stage).  nullptr: takes back one not yet used.
-bool demag_take_stage(DemagBase *d, const void *stage);
 void demag_destroy(DemagBase *d);
 void demag_kspec(DemagBase *d, int c, void *host);
 void demag_info(DemagBase *d, int P[3], int *prec);
