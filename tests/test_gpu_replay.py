@@ -74,3 +74,18 @@ def test_batched_chains(gpu):
             s.steps(n)
         for i in range(30):
             _same(alone[i], batch[i], (i, n))
+
+
+def test_batched_skewed_ensemble(gpu):
+    """One member with more than half of the work among 48: its share of the
+    cost skips whole chains, which must not be kept without members."""
+    for big in (0, 24, 47):
+        print("skewed ensemble", big, flush=True)
+        make = lambda i, g: _sim(gpu, (512, 512, 1) if i == big else ((64, 64, 1), (60, 64, 1))[i % 2], i, "heun", g)
+        alone, batch = ([make(i, g) for i in range(48)] for g in (0, 1))
+        for n in (4, 5):
+            gpu.sims_steps_batched(batch, n)
+            for s in alone:
+                s.steps(n)
+            for i in range(48):
+                _same(alone[i], batch[i], (big, i, n))

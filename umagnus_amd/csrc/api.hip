@@ -1194,6 +1194,10 @@ static BatchPlan *batch_plan_build(const std::vector<SimBase *> &m) {
     P->chains[std::min(nc - 1, (int)((before + 0.5 * cost[i]) * nc / all))].members.push_back(i);
     before += cost[i];
   }
+  // a member with more than a chain's share of the work leaves chains empty
+  P->chains.erase(std::remove_if(P->chains.begin(), P->chains.end(),
+                                 [](const BatchChain &c) { return c.members.empty(); }),
+                  P->chains.end());
   std::vector<size_t> head(nm, 0);
   std::vector<unsigned char> host;
   auto put = [&](const void *p, size_t bytes) {
@@ -1369,7 +1373,7 @@ int um_sims_steps_batched(int nsims, void *const *sims, int n, int *launches_per
           }
         for (long r = 0; r < R; r++) {
           for (BatchChain &ch : P->chains)
-            if (ch.gexec) UM_HIP(hipGraphLaunch(ch.gexec, ch.st));
+            UM_HIP(hipGraphLaunch(ch.gexec, ch.st));
           for (SimBase *x : mem) x->batch_advance();
         }
         for (BatchChain &ch : P->chains) {
