@@ -475,7 +475,8 @@ int um_sims_steps(int nsims, void *const *sims, int n);
  * work-group working on its own member's grid and buffers, so each member
  * computes what it computes alone (um_sims_steps, um_sim_steps), bit for bit.
  * The merged sequences are replayed as graphs of two steps; they are rebuilt
- * when a member's parameters, solver, FixDt or buffers change.  Members not in
+ * when a member's parameters, solver, FixDt or buffers change (two steps of a
+ * few changed members run eagerly instead).  Members not in
  * graph mode with FixDt step eagerly in turn.  *launches_per_two_steps (when
  * not NULL) receives the number of launches that replay two steps of the
  * whole ensemble, or 0 when a member needs a kernel without a batched form

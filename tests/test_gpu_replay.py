@@ -89,3 +89,25 @@ def test_batched_skewed_ensemble(gpu):
                 s.steps(n)
             for i in range(48):
                 _same(alone[i], batch[i], (big, i, n))
+
+
+def test_batched_two_steps_of_changed_members(gpu):
+    """Two steps of a few changed members are not worth a new plan; the second
+    such call on unchanged members is, and so are two steps of many."""
+    def launches(sims, n):
+        with gpu.KernelTrace() as tr:
+            gpu.sims_steps_batched(sims, n)
+        return sum("k_batch" in k for k in tr.names)
+
+    alone, batch = ([_sim(gpu, (nx, 20, 1), i, "heun", g)
+                     for i, nx in enumerate((32, 36, 40, 42, 48, 50, 54, 56))] for g in (0, 1))
+    for count, builds in ((3, (False, True, False, False)), (8, (True, False, False, True))):
+        for call, build in enumerate(builds):
+            print("two steps", count, call, flush=True)
+            if call in (0, 3):
+                for s in alone[:count] + batch[:count]:
+                    s.set_vector(gpu.P_BEXT, (0.01 * (call + count), 0.0, 0.0))
+            assert (launches(batch[:count], 2) > 0) == build, (count, call)
+            for i, s in enumerate(alone[:count]):
+                s.steps(2)
+                _same(s, batch[i], (count, call, i))

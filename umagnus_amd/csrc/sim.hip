@@ -1210,10 +1210,11 @@ struct Sim : SimBase {
     for (int i = 0; i < 8 && fresh; i++) fresh = (g_ptrs[i] == ptrs[i]);
     if (!fresh) capture2();
   }
-  long batch_prepare(long stop) override { return prepare_replays(stop, false); }
-  long prepare_replays(long stop, bool capture) {
+  bool batch_usable() const override { return graph_usable(); }
+  long batch_prepare(long stop, bool replay) override { return prepare_replays(stop, false, replay); }
+  long prepare_replays(long stop, bool capture, bool replay = true) {
     k1_valid = false;
-    if (!graph_usable() || nsteps >= stop) return 0;
+    if (!replay || !graph_usable() || nsteps >= stop) return 0;
     if (nsteps + 2 > stop) return 0;
     // A captured step computes what an eager one does, so the replays may start
     // at once: they need the plan, the FSAL torque of the solvers that keep one,

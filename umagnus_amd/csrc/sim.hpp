@@ -94,11 +94,13 @@ struct SimBase {
   virtual void set_profiling(int on) = 0;
   virtual void set_graph(int on) = 0;
   virtual long graph_prepare(long stop) = 0;
-  // batched ensembles: as graph_prepare without capturing a graph; then the
+  // batched ensembles: whether fixed-dt steps can be replayed; as
+  // graph_prepare without capturing a graph (replay false: no replays); the
   // launches of two fixed-dt steps recorded instead of run (batch.hpp),
   // a key that changes whenever such a recording would, and the host side
   // of two replayed steps
-  virtual long batch_prepare(long stop) = 0;
+  virtual bool batch_usable() const = 0;
+  virtual long batch_prepare(long stop, bool replay) = 0;
   virtual void graph_ensure() = 0;   // capture the two-step graph if it is stale
   virtual void batch_record(std::vector<struct BatchEntry> &out) = 0;
   virtual std::vector<uint64_t> batch_key() const = 0;
