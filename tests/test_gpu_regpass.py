@@ -72,3 +72,29 @@ def test_register_passes_vs_oracle(gpu, oracle, N, pbc, prec):
         ref = od.exec(m, np.full(shape, ms) if np.isscalar(ms) else ms, vol=v)
         err = np.abs(got - ref).max() / np.abs(ref).max()
         assert err < (1e-12 if prec == 1 else 2e-6), (N, pbc, prec, err)
+
+
+# periodic z: dense columns in registers (FP32, 2..8 and 16 points, the latter
+# from 24576 columns) and in LDS (9, 16 below that, FP64); odd column counts,
+# rows with and without a mirror
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("N,pbc", [((10, 6, 2), (0, 0, 1)), ((35, 7, 3), (0, 0, 2)), ((30, 5, 4), (1, 0, 1)),
+                                   ((12, 9, 5), (0, 0, 1)), ((9, 4, 6), (1, 1, 1)), ((70, 6, 7), (0, 0, 1)),
+                                   ((20, 7, 8), (0, 1, 1)), ((12, 10, 9), (0, 0, 1)), ((20, 12, 16), (0, 0, 1)),
+                                   ((126, 98, 16), (0, 0, 1))])
+def test_periodic_z_vs_oracle(gpu, oracle, N, pbc, prec):
+    test_register_passes_vs_oracle(gpu, oracle, N, pbc, prec)
+
+
+def test_periodic_z_kernels(gpu):
+    """FP32 dense columns run in registers from 2 to 8 points and, with enough
+    columns, of 16."""
+    import torch
+    for N, short in (((64, 8, 3), True), ((32, 8, 8), True), ((32, 8, 9), False), ((32, 8, 16), False),
+                     ((128, 96, 16), True)):
+        m = [torch.ones(N[2], N[1], N[0], device="cuda") for _ in range(3)]
+        B = [torch.zeros_like(x) for x in m]
+        conv = gpu.DemagConvolution(N, (2e-9,) * 3, pbc=(0, 0, 1), precision=0)
+        with gpu.KernelTrace() as tr:
+            conv.Exec(B, m, None, 8e5)
+        assert any("k_rshort" in k for k in tr.names) == short, (N, tr.names)

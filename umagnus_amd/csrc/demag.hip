@@ -1824,7 +1824,7 @@ struct DemagPlan : DemagBase {
     const int nx = P[0] / 2, ny = P[1], convlen = is2d ? P[1] : P[2];
     if (!xodd && !CtTable<T>::x(nx) && !x4_ok<T>(nx, N[0])) rx.append(REG_X, nx, (long)N[1] * N[2], 3, roots, h);
     if (!is2d && !coly_len<T>(ny)) ry.append(REG_COL, ny, H, 3L * N[2], roots, h);
-    rshort = !is2d && short_ok<T>(N[2], P[2]);
+    rshort = !is2d && short_ok<T>(N[2], P[2], (long)H * P[1]);
     if (!rshort && !zreg && !CtTable<T>::conv(convlen, is2d, H))
       rc.append(REG_CONV, convlen, H, is2d ? 1L : (long)P[1], roots, h);
     if (h.empty()) return;
@@ -2015,7 +2015,7 @@ struct DemagPlan : DemagBase {
       r.H = k.n; r.Py = P[1]; r.KHy = KHy; r.Hk = Hk; r.zstride = (long)P[1] * Hp; r.ystride = Hp;
       for (int c = 0; c < 6; c++) r.K[c] = K[c];
       for (int c = 0; c < 3; c++) r.buf[c] = spec[c].as<C2<T>>() + k.x0;
-      launch_rshort<T>(r, N[2], s);
+      launch_rshort<T>(r, N[2], P[2], s);
       return;
     }
     if (rc.len.n && (is2d ? ty : tz).sched == 0) {

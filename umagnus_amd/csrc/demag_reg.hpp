@@ -116,7 +116,8 @@ template <typename T> void launch_rxinv(const RXArgs<T> &a, int nt, hipStream_t 
 template <typename T> void launch_rxstage(const RXStageArgs<T> &a, int nt, hipStream_t s);
 template <typename T> void launch_rcol(const RColArgs<T> &a, int dir, int planes, int nt, hipStream_t s);
 template <typename T> void launch_rconv(const RConvArgs<T> &a, int nt, hipStream_t s);
-template <typename T> bool short_ok(int Nz, int Pz);
-template <typename T> void launch_rshort(const RShortArgs<T> &a, int Nz, hipStream_t s);
+// register z columns: columns = kx columns times ky rows
+template <typename T> bool short_ok(int Nz, int Pz, long columns);
+template <typename T> void launch_rshort(const RShortArgs<T> &a, int Nz, int Pz, hipStream_t s);
 
 }  // namespace um

@@ -537,9 +537,13 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 4 : 1) void k_rconv(RConvArgs
 // One thread per (kx, ky) column, the three components in registers, no LDS.
 // Pz = 2 Nz: the even and odd frequencies are two Nz-point transforms
 //   X[2m] = DFT(x)[m], X[2m+1] = DFT(x W_Pz^n)[m],
-// multiplied and transformed back one after the other; Pz = 2 Nz - 1 (Nz <= 5):
-// one Pz-point transform.  160 x 160 x 10 FP32: 93.8 -> 11.8 us (32 MB),
+// multiplied and transformed back one after the other; Pz = 2 Nz - 1 (Nz <= 5)
+// and Pz = Nz (periodic z): one Pz-point transform.  160 x 160 x 10 FP32: 93.8 -> 11.8 us (32 MB),
 // 320 x 200 x 6: 166 -> 11.6, against the generic convolution kernel.
+// Periodic z in FP32, a whole convolution with k_rconv -> with this: 128 x 128
+// x 3 26.3 -> 21.5 us, x 7 38.4 -> 28.0, 512 x 512 x 7 272 -> 121, x 16 336 ->
+// 268; 16 points need many columns to hide a thread's chain (128 x 96 x 16,
+// 24768 columns, 40.5 -> 40.1; 96 x 96 x 16, 18624, 33.8 -> 38.6).
 // A wave holds 32 kx of ky (lanes 0-31) and of its
 // mirror Py - ky (lanes 32-63), which read the same tensor lines.
 template <typename T, int NZ, int PZ>
@@ -664,10 +668,22 @@ void launch_rconv(const RConvArgs<T> &a, int nt, hipStream_t s) {
   UM_HIP(hipGetLastError());
 }
 template <typename T>
-void launch_rshort(const RShortArgs<T> &a, int Nz, hipStream_t s) {
+void launch_rshort(const RShortArgs<T> &a, int Nz, int Pz, hipStream_t s) {
   const dim3 grid((a.H + 31) / 32, (a.KHy + 3) / 4);
 #define UM_RSHORT(NZ, PZ) \
   case NZ: launch_b<BRShort<T, NZ, PZ>>(k_rshort<T, NZ, PZ>, grid, dim3(256), 0, s, a); break;
+  if (Pz == Nz) {
+    if constexpr (sizeof(T) == 4) {
+      switch (Nz) {
+        UM_RSHORT(2, 2) UM_RSHORT(3, 3) UM_RSHORT(4, 4) UM_RSHORT(5, 5) UM_RSHORT(6, 6) UM_RSHORT(7, 7)
+        UM_RSHORT(8, 8) UM_RSHORT(16, 16)
+        default: throw Error(UM_EUNSUP, "register z columns: unsupported Nz");
+      }
+      UM_HIP(hipGetLastError());
+      return;
+    }
+    throw Error(UM_EUNSUP, "register z columns: unsupported Nz");
+  }
   switch (Nz) {
     UM_RSHORT(2, 3) UM_RSHORT(3, 5) UM_RSHORT(4, 7) UM_RSHORT(5, 9) UM_RSHORT(6, 12) UM_RSHORT(7, 14)
     default:
@@ -684,7 +700,8 @@ void launch_rshort(const RShortArgs<T> &a, int Nz, hipStream_t s) {
   UM_HIP(hipGetLastError());
 }
 template <typename T>
-bool short_ok(int Nz, int Pz) {
+bool short_ok(int Nz, int Pz, long columns) {
+  if (Pz == Nz) return sizeof(T) == 4 && Nz >= 2 && (Nz <= 8 || (Nz == 16 && columns >= 24576));
   if (Nz >= 2 && Nz <= 5) return Pz == 2 * Nz - 1;
   if (Pz != 2 * Nz) return false;
   return Nz == 6 || Nz == 7 || (sizeof(T) == 4 && (Nz == 9 || Nz == 10 || Nz == 12));
@@ -717,8 +734,8 @@ void RegTab<T>::bind(const C2<T> *dev) {
   template void launch_rxstage<T>(const RXStageArgs<T> &, int, hipStream_t); \
   template void launch_rcol<T>(const RColArgs<T> &, int, int, int, hipStream_t); \
   template void launch_rconv<T>(const RConvArgs<T> &, int, hipStream_t);   \
-  template void launch_rshort<T>(const RShortArgs<T> &, int, hipStream_t); \
-  template bool short_ok<T>(int, int);                                     \
+  template void launch_rshort<T>(const RShortArgs<T> &, int, int, hipStream_t); \
+  template bool short_ok<T>(int, int, long);                               \
   template struct RegTab<T>;
 
 }  // namespace um
