@@ -2039,30 +2039,38 @@ struct DemagPlan : DemagBase {
     launch_conv<T>(ca, is2d ? P[1] : P[2], B_conv, gc, s);
   }
   // Columns per run of the Y forward, Z and Y inverse passes.  A spectrum that
-  // exceeds the 256 MB last-level cache is taken in parts of at most 208 MB, so
-  // that a pass finds in the cache what the pass before it wrote (the cache
-  // moves 8.5 TB/s, HBM 5 to 6).  Convolution of 1024 x 1024 x 8 FP32 (403 MB)
-  // whole 767 us, in 2 parts 710; x 16 1538, 4 parts 1399; x 32 3010, 8 parts
-  // 2843; 400 x 400 x 40 804, 2 parts 783; 2000 x 1000 x 10 the same.  What fits
-  // gains nothing and fills its last round of work-groups worse (512 x 512 x 16,
-  // 202 MB: 277, 2 parts 293).  k_coly's lengths stay whole, one launch per pass:
-  // their wide tiles leave a gain at few of the sizes (512 x 512 x 32: 587, 2
-  // parts 562, 3 parts 595, 6 parts 692).  FP64 passes are bound by their
-  // arithmetic (512 x 512 x 32 1497, 4 parts 1535): never split.  Parts start on
-  // a 256-byte boundary of the rows.
-  int chunk_cols() const {
-    if (sizeof(T) != 4 || !ry.len.n || ty.sched != 0) return H;
-    const int parts = (int)ceil(3.0 * sizeof(C2<T>) * N[2] * P[1] * H / 208e6);
-    return parts > 1 ? std::max(32, (H / parts + 31) / 32 * 32) : H;
+  // exceeds the 256 MB last-level cache is taken in parts of at most 208 MB (the
+  // last one 240 MB, so that it takes up a narrow rest), so that a pass finds in
+  // the cache what the pass before it wrote (the cache moves 8.5 TB/s, HBM 5 to
+  // 6).  Convolution of 1024 x 1024 x 8 FP32 (403 MB) whole 767 us, in 2 parts
+  // 710; x 16 1538, 4 parts 1399; x 32 3010, 8 parts 2843; 400 x 400 x 40 804, 2
+  // parts 783.  What fits gains nothing and fills its last round of work-groups
+  // worse (512 x 512 x 16, 202 MB: 277, 2 parts 293), and so do narrow parts of
+  // deep columns: 96 columns (fewer gain nothing in any grid) pay where the Z
+  // pass runs in registers (525 x 1000 x 32 1853, parts of 128 1825; 320 x 1080
+  // x 32 1176, parts of 96 1167), 128 where it is k_rconv (500 x 800 x 36 1841,
+  // 1791; 1000 x 640 x 40 3130, 3084; 800 x 1000 x 40 4155, parts of 96 4244;
+  // 60 x 2000 x 64 1272, parts of 32 1300).  k_coly's lengths stay whole, one
+  // launch per pass: their wide tiles leave a gain at few of the sizes (512 x
+  // 512 x 32: 587, 2 parts 562, 3 parts 595, 6 parts 692).  FP64 passes are
+  // bound by their arithmetic (512 x 512 x 32 1497, 4 parts 1535): never split.
+  // Parts start on a 256-byte boundary of the rows.
+  struct Parts { int w, last; };   // columns of a part, and at most of the last one
+  Parts parts() const {
+    if (sizeof(T) != 4 || !ry.len.n || ty.sched != 0) return {H, H};
+    const double col = 3.0 * sizeof(C2<T>) * N[2] * P[1];
+    const int np = (int)ceil(col * H / 208e6), fit = (int)(208e6 / col) / 32 * 32;
+    if (np < 2 || fit < (rc.len.n ? 128 : 96)) return {H, H};
+    return {std::min(fit, (H / np + 31) / 32 * 32), (int)(240e6 / col)};
   }
   // X forward through Y inverse (3D) or the 2D Y pass: leaves the convolved
   // half spectrum (rows y < Ny) in spec[] for the X inverse.
   void spectral(const void *const mv[3], const void *vol, const void *Msa, double Ms_mul, hipStream_t s,
                 const StageArgs<T> *stage = nullptr) {
     pass_xfwd(mv, vol, Msa, Ms_mul, s, stage);
-    const int w = chunk_cols();
+    const Parts p = parts();
     for (Cols k{0, 0}; k.x0 < H; k.x0 += k.n) {
-      k.n = H - k.x0 <= w + w / 4 ? H - k.x0 : w;
+      k.n = H - k.x0 <= p.last ? H - k.x0 : p.w;
       if (!is2d) pass_y(-1, k, s);
       pass_conv(k, s);
       if (!is2d) pass_y(+1, k, s);
