@@ -274,7 +274,8 @@ int um_demag_kernel_newell(int Nx, int Ny, int Nz, const int pbc[3], const doubl
  * every new shape when its plan is created (results kept per precision and
  * size until the next call); 2: apply known results only.  file (or NULL):
  * the known results are read from it now and new ones appended, so later
- * processes reuse them. */
+ * processes reuse them.  Entries that an earlier version of the kernels wrote
+ * are timed again by mode 1 and applied as they are by mode 2. */
 int um_set_autotune(int mode, const char *file);
 /* the schedule of a plan: nl_x nl_xi four_step nl_y B_conv sched_x sched_y sched_z */
 int um_demag_schedule(void *plan, int out[8]);

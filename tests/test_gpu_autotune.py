@@ -94,3 +94,27 @@ def test_tuned_plans(gpu, oracle, tmp_path, N, pbc, prec):
         assert len(f.read_text().splitlines()) == 1
     finally:
         gpu.set_autotune(0)
+
+
+def test_entries_without_generation(gpu, oracle, tmp_path):
+    """An entry without a generation mark, whose schedules meant other kernels:
+    tuned again in mode 1 and written with the mark; applied in mode 2."""
+    N = (60, 50, 3)
+    f = tmp_path / "old.txt"
+    old = "%s: 4 4 1 4 4 2 2 2\n" % _key(oracle, N, (0, 0, 0), 0)
+    f.write_text(old)
+    try:
+        gpu.set_autotune(2, str(f))
+        assert _check(gpu, oracle, N, (0, 0, 0), 0) == [4, 4, 1, 4, 4, 2, 2, 2]
+        assert f.read_text() == old
+        gpu.set_autotune(1, str(f))
+        sched = _check(gpu, oracle, N, (0, 0, 0), 0)
+        lines = f.read_text().splitlines()
+        assert len(lines) == 2 and lines[1] == "%s: %s : 2" % (old.split(":")[0], " ".join(map(str, sched)))
+        # the marked entry is the one that counts from now on, in both modes
+        for mode in (1, 2):
+            gpu.set_autotune(mode, str(f))
+            assert _check(gpu, oracle, N, (0, 0, 0), 0) == sched
+            assert len(f.read_text().splitlines()) == 2
+    finally:
+        gpu.set_autotune(0)

@@ -1676,10 +1676,18 @@ struct DemagBase {
 // read back by later calls and processes.  Off by default: the static tables are then used, and results do
 // not depend on timing noise.  Mode 2 applies known results (from the
 // file) without timing anything.
+//
+// An entry is "key: knobs : generation".  The generation changes with what the
+// knobs select: in entries without one schedule 0 was the Stockham engine's
+// default order, so their schedules 1 to 3 may shut off register passes that
+// are several times faster.  Mode 1 times such shapes again; mode 2, which
+// also takes entries written by hand, applies them and says so.
+constexpr int TUNE_GEN = 2;
+struct TuneEntry { std::vector<int> v; int gen; };
 static std::mutex g_tune_mu;
 static int g_tune_mode = 0;
 static std::string g_tune_file;
-static std::map<std::string, std::vector<int>> g_tune_memo;
+static std::map<std::string, TuneEntry> g_tune_memo;
 
 void set_autotune(int mode, const char *file) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -1702,7 +1710,9 @@ void set_autotune(int mode, const char *file) {
       v.push_back((int)x);
       q = end;
     }
-    if ((int)v.size() == DEMAG_NKNOB) g_tune_memo[std::string(line, colon)] = v;
+    const char *mark = std::strchr(q, ':');
+    const int gen = mark ? (int)std::strtol(mark + 1, nullptr, 10) : 1;
+    if ((int)v.size() == DEMAG_NKNOB) g_tune_memo[std::string(line, colon)] = TuneEntry{v, gen};
   }
   std::fclose(f);
 }
@@ -1711,17 +1721,25 @@ static bool tune_lookup(const std::string &key, std::vector<int> &v, int *mode) 
   *mode = g_tune_mode;
   auto it = g_tune_memo.find(key);
   if (it == g_tune_memo.end()) return false;
-  v = it->second;
+  v = it->second.v;
+  if (it->second.gen == TUNE_GEN) return true;
+  if (*mode != 2) return false;
+  static bool said = false;
+  if (!said && (v[5] || v[6] || v[7])) {
+    said = true;
+    fprintf(stderr, "umhip: the tuning file's entry \"%s\" has no generation mark and shuts off register passes; "
+                    "remove it or tune again (mode 1)\n", key.c_str());
+  }
   return true;
 }
 static void tune_store(const std::string &key, const std::vector<int> &v) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune_memo[key] = v;
+  g_tune_memo[key] = TuneEntry{v, TUNE_GEN};
   if (g_tune_file.empty()) return;
   if (FILE *f = std::fopen(g_tune_file.c_str(), "a")) {
     std::fprintf(f, "%s:", key.c_str());
     for (int x : v) std::fprintf(f, " %d", x);
-    std::fprintf(f, "\n");
+    std::fprintf(f, " : %d\n", TUNE_GEN);
     std::fclose(f);
   }
 }
