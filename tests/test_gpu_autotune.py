@@ -96,6 +96,29 @@ def test_tuned_plans(gpu, oracle, tmp_path, N, pbc, prec):
         gpu.set_autotune(0)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("N", [(100, 100, 2), (250, 250, 1), (64, 64, 8), (90, 80, 15)])
+def test_no_choice_among_equals(gpu, oracle, tmp_path, N, prec):
+    """A pass that ignores the rows or columns knob (register passes at schedule
+    0, four-step X, register Y of 64 and 256) keeps its static value: tuning
+    does not pick one of many timings of the same kernel."""
+    _say("equals", N, prec)
+    gpu.set_autotune(0)
+    base = _check(gpu, oracle, N, (0, 0, 0), prec)
+    gpu.set_autotune(1, str(tmp_path / "tune.txt"))
+    try:
+        got = _check(gpu, oracle, N, (0, 0, 0), prec)
+    finally:
+        gpu.set_autotune(0)
+    assert got[2] == base[2] == 1
+    if got[5] == 0:
+        assert got[:2] == base[:2]
+    if got[6] == 0:
+        assert got[3] == base[3]
+    if got[6 if N[2] == 1 else 7] == 0:
+        assert got[4] == base[4]
+
+
 def test_entries_without_generation(gpu, oracle, tmp_path):
     """An entry without a generation mark, whose schedules meant other kernels:
     tuned again in mode 1 and written with the mark; applied in mode 2."""

@@ -2182,6 +2182,12 @@ struct DemagPlan : DemagBase {
     return B >= 1 && B * (convlen / 2 + 1) <= FFT_NT * CONV_QK && 3 * B * convlen <= FFT_NT * FftEpt<T>::value;
   }
 
+  // Only candidates that run different kernels or grids are timed: the register
+  // passes (schedule 0) and the compiled lengths ignore the other knobs, and a
+  // choice among equals would store noise.  first: the static choice.
+  static bool differs(bool reg, bool compiled, bool first, int sc) {
+    return compiled ? sc == 0 : reg && sc == 0 ? first : true;
+  }
   void tune(hipStream_t s) override {
     const std::string key = tune_key();
     std::vector<int> v;
@@ -2226,9 +2232,11 @@ struct DemagPlan : DemagBase {
     try {
       spectral(mv, nullptr, nullptr, 1.0, s);   // valid spectra in the buffers
       // 1. X forward: rows per work-group x radix schedule
-      {
+      const int nx = xodd ? P[0] : P[0] / 2;
+      const bool x4 = !xodd && x4_ok<T>(nx, N[0]);
+      if (!(x4 && xi4)) {
         std::vector<int> nls;
-        const int nx = xodd ? P[0] : P[0] / 2;
+        const int ct = xodd ? 0 : CtTable<T>::x(nx);
         add(nls, nl_x);
         if (!xodd && std::is_same<T, float>::value && CtTable<T>::x(nx)) {
           add(nls, CtTable<T>::x(nx));
@@ -2240,6 +2248,7 @@ struct DemagPlan : DemagBase {
         int bn = nl_x, bs = xtab().sched;
         for (int nl : nls)
           for (int sc = 0; sc < FFT_NSCHED; sc++) {
+            if (!differs(rx.len.n, ct && (nl == ct || nl == ct / 4 || nl == 1), nl == nls[0], sc)) continue;
             nl_x = nl;
             try { xtab().schedule(sc); } catch (const Error &) { continue; }   // too many passes
             const float t = timed([&] { pass_xfwd(mv, nullptr, nullptr, 1.0, s); });
@@ -2250,7 +2259,6 @@ struct DemagPlan : DemagBase {
       }
       // 2. X inverse: four-step kernel or the Stockham one with rows per work-group
       {
-        const int nx = xodd ? P[0] : P[0] / 2;
         std::vector<int> nls;
         add(nls, nl_xi);
         if (!xodd && CtTable<T>::x(nx)) add(nls, CtTable<T>::x(nx));
@@ -2260,7 +2268,8 @@ struct DemagPlan : DemagBase {
         bool b4 = xi4;
         for (int four : {1, 0})
           for (int nl : nls) {
-            if (four && nl != nls[0]) continue;   // the four-step kernel has its own rows
+            if (x4 && four && nl != nls[0]) continue;   // the four-step kernel has its own rows
+            if (!x4 && (four != (int)b4 || !differs(rx.len.n, false, nl == nls[0], tx.sched))) continue;
             xi4 = four != 0;
             nl_xi = nl;
             const float t = timed([&] { pass_xinv(bv, s); });
@@ -2270,7 +2279,7 @@ struct DemagPlan : DemagBase {
         xi4 = b4;
       }
       // 3. Y passes (3D): generic lines per work-group x radix schedule
-      if (!is2d) {
+      if (!is2d && !coly_len<T>(P[1])) {
         std::vector<int> nls;
         add(nls, nl_y);
         for (int x : halvings(std::min(lines_for(P[1]), 64))) add(nls, x);
@@ -2278,6 +2287,7 @@ struct DemagPlan : DemagBase {
         int bn = nl_y, bs = ty.sched;
         for (int nl : nls)
           for (int sc = 0; sc < FFT_NSCHED; sc++) {
+            if (!differs(ry.len.n, false, nl == nls[0], sc)) continue;
             nl_y = nl;
             try { ty.schedule(sc); } catch (const Error &) { continue; }
             const float t = timed([&] { const Cols k{0, H}; pass_y(-1, k, s); pass_y(+1, k, s); });
@@ -2299,6 +2309,7 @@ struct DemagPlan : DemagBase {
         for (int B : bs_) {
           if (!conv_ok(B)) continue;
           for (int sc = 0; sc < FFT_NSCHED; sc++) {
+            if (!differs(rshort || rc.len.n, B == CtTable<T>::conv(convlen, is2d, H), B == bs_[0], sc)) continue;
             B_conv = B;
             try { tc.schedule(sc); } catch (const Error &) { continue; }
             const float t = timed([&] { pass_conv({0, H}, s); });
