@@ -187,3 +187,23 @@ def test_time_function_switches_demag(gpu, monkeypatch, dtype):
         out.append(np.array(s.get_m()))
     assert np.array_equal(*out)
     assert np.abs((out[0].astype(float) ** 2).sum(0) - 1).max() < 1e-6
+
+
+def test_profiled_steps_keep_stages_apart(gpu):
+    """The demag share of um_sim_kernel_times holds no solver stage; profiled
+    steps give the same bits."""
+    N, out = (30, 20, 3), []
+    for profiling in (0, 1):
+        s = gpu.Sim(N, (4e-9, 3e-9, 2e-9), dtype=np.float32)
+        s.set_scalar(gpu.P_MSAT, 8e5)
+        s.set_scalar(gpu.P_ALPHA, 0.1)
+        s.set_exchange_luts(exchange_lut(1.3e-11, dtype=np.float32), None)
+        s.set_m(random_unit((3, 20, 30), 8).astype(np.float32))
+        s.set_solver(5)
+        s.set_solver_params(dt=1e-13, fixdt=1e-13)
+        s.set_profiling(profiling)
+        with gpu.KernelTrace() as tr:
+            s.steps(2)
+        assert any("k_rxstage" in k for k in tr.names) == (not profiling), tr.names
+        out.append(np.array(s.get_m()))
+    assert np.array_equal(*out)

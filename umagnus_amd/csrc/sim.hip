@@ -647,11 +647,12 @@ struct Sim : SimBase {
   // a stage into m and the torque of the result: the demag plan may form m in
   // its X forward pass.  Not with time functions: torque_fn calls them before
   // the convolution is enqueued, and they may read m (get_m, average_m,
-  // m_device), which must then hold the stage.
+  // m_device), which must then hold the stage.  Nor while profiling, whose demag
+  // share is the convolution's alone.
   void stage_torque(int ns, const T *const *src, const T *fac, bool norm, bool group3, T *kout) {
     const StageArgs<T> a = stage_args(m, ns, src, fac, norm, group3, nullptr);
     bool taken = false;
-    if (enable_demag && !has_nodemag && !any_tfn && !xterm_tfn) {
+    if (enable_demag && !has_nodemag && !any_tfn && !xterm_tfn && !profiling) {
       ensure_demag();
       taken = demag_takes_stage(demag, &a);
     }
