@@ -141,3 +141,39 @@ def test_entries_without_generation(gpu, oracle, tmp_path):
             assert len(f.read_text().splitlines()) == 2
     finally:
         gpu.set_autotune(0)
+
+
+# lengths without a register split: X rows (FP64 has fewer radices), Y columns,
+# the film's and the z axis' convolution
+STOCKHAM = [((625, 4, 2), 0, ("k_xfwd", "k_xinv")), ((625, 4, 2), 1, ("k_xfwd", "k_xinv")),
+            ((375, 6, 1), 1, ("k_xfwd", "k_xinv")), ((784, 3, 1), 1, ("k_xfwd", "k_xinv")),
+            ((4, 625, 2), 0, ("k_colfft",)), ((4, 625, 2), 1, ("k_colfft",)),
+            ((6, 625, 1), 0, ("k_conv",)), ((6, 625, 1), 1, ("k_conv",)),
+            ((3, 2, 625), 0, ("k_conv",)), ((3, 2, 625), 1, ("k_conv",))]
+
+
+@pytest.mark.parametrize("N,prec,kernels", STOCKHAM)
+def test_lengths_of_the_stockham_engine(gpu, oracle, tmp_path, N, prec, kernels):
+    """The run-time Stockham engine at every schedule, where it is the pass of
+    the length: the static plan (schedule 0) launches it."""
+    gpu.set_autotune(0)
+    base = _check(gpu, oracle, N, (0, 0, 0), prec)
+    dt = np.float32 if prec == 0 else np.float64
+    m = [_t(np.ones((N[2], N[1], N[0])), dt) for _ in range(3)]
+    B = [_t(np.zeros((N[2], N[1], N[0])), dt) for _ in range(3)]
+    conv = gpu.DemagConvolution(N, (2e-9, 3e-9, 2.5e-9), precision=prec)
+    with gpu.KernelTrace() as tr:
+        conv.Exec(B, m, None, 8e5)
+    assert base[5:] == [0, 0, 0]
+    for k in kernels:
+        assert any("um::%s<" % k in name for name in tr.names), (k, tr.names)
+    for sc in (1, 2, 3):
+        _say("stockham", N, prec, sc)
+        f = tmp_path / ("s%d.txt" % sc)
+        v = base[:5] + [sc, sc, sc]
+        f.write_text("%s: %s\n" % (_key(oracle, N, (0, 0, 0), prec), " ".join(map(str, v))))
+        gpu.set_autotune(2, str(f))
+        try:
+            assert _check(gpu, oracle, N, (0, 0, 0), prec) == v
+        finally:
+            gpu.set_autotune(0)
