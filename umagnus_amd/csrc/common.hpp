@@ -12,6 +12,8 @@
 
 namespace um {
 
+constexpr double MU0 = 4 * 3.14159265358979323846 * 1e-7;   // mag/constants.go:8
+
 // ---- errors ----------------------------------------------------------------
 struct Error : std::runtime_error {
   int code;

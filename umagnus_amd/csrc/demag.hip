@@ -32,8 +32,6 @@
 
 namespace um {
 
-static constexpr double MU0 = 4 * M_PI * 1e-7;
-
 // Data movement between HBM and LDS uses fixed-trip, fully unrolled slots
 // (slot s of thread t handles flat index g = t + s*FFT_NT, g < nl*n <= FFT_NT*EPT)
 // so every global load of a work-group is in flight before the first LDS store.
@@ -1557,8 +1555,7 @@ static void launch_xfwd(const XArgs<T> &a, int n, int nl, dim3 grid, hipStream_t
   UM_HIP(hipGetLastError());
 }
 template <typename T>
-static void launch_xinv(const XiArgs<T> &a, int n, int nl, dim3 grid, hipStream_t s, bool four_step = true) {
-  if (four_step && launch_xi4<T>(a, n, s)) return;
+static void launch_xinv(const XiArgs<T> &a, int n, int nl, dim3 grid, hipStream_t s) {
   const size_t ct = sizeof(C2<T>) * ((size_t)nl * n + 2 * n);
   if constexpr (std::is_same<T, float>::value) {
     UM_CT_CASE((BXinv<float, 32, 32>), (k_xinv<float, 32, 32>), 32, 32, ct)
@@ -2109,7 +2106,7 @@ struct DemagPlan : DemagBase {
         r.pairs = even_pairs(r.dst, nullptr, nullptr);
         launch_rxinv<T>(r, rx.nt, s);
       } else {
-        launch_xinv<T>(a, P[0] / 2, nl_xi, g, s, false);
+        launch_xinv<T>(a, P[0] / 2, nl_xi, g, s);
       }
     }
   }

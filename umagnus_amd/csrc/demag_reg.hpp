@@ -6,7 +6,7 @@
 // and a line crosses LDS once per stage boundary.  The frequency of slot
 // (k0, k1, j) is k0 + r0 k1 + r0 r1 j; nothing is reordered in memory.
 //
-// Host side: reg_len() picks the radices, launch_r*() run a pass.
+// Host side: reg_plan() picks the radices, launch_r*() run a pass.
 #pragma once
 #include <map>
 #include <vector>

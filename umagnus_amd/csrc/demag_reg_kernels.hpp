@@ -6,8 +6,6 @@
 
 namespace um {
 
-static constexpr double MU0_R = 4 * M_PI * 1e-7;
-
 // a stage body called out of line would keep its captures in scratch memory
 #define UM_INLINE __attribute__((always_inline))
 template <int R> struct RadixTag { static constexpr int value = R; };
@@ -127,7 +125,7 @@ struct BRXfwd {
     const T *src = pick(a.src, c);
     C2<T> *out = pick(a.spec, c);
     const T *const msa = a.Ms.arr, *const vol = a.vol;
-    const T mul = a.Ms.mul, fac = T(MU0_R) * mul;
+    const T mul = a.Ms.mul, fac = T(MU0) * mul;
     with_radix<RegMax<T>::X>(f.r[0], [&](auto tag) UM_INLINE {
       constexpr int R = decltype(tag)::value;
       for (int g = threadIdx.x; g < nl * f.n1; g += blockDim.x) {
@@ -160,7 +158,7 @@ struct BRXfwd {
           if (msa) {
             row(msa, w);
 #pragma unroll
-            for (int j = 0; j < R; j++) w[j] = C2<T>{T(MU0_R) * (mul * w[j].x), T(MU0_R) * (mul * w[j].y)};
+            for (int j = 0; j < R; j++) w[j] = C2<T>{T(MU0) * (mul * w[j].x), T(MU0) * (mul * w[j].y)};
           } else {
 #pragma unroll
             for (int j = 0; j < R; j++) w[j] = C2<T>{fac, fac};

@@ -1,4 +1,5 @@
-// Device side of the LDS Stockham FFT engine (included by demag.hip only).
+// Device side of the LDS Stockham FFT engine and the register transforms of the
+// other FFT passes.
 #pragma once
 #include "fft.hpp"
 

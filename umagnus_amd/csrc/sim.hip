@@ -17,7 +17,6 @@
 namespace um {
 
 static constexpr double KB = 1.380650424e-23;  // mag/constants.go:9
-static constexpr double MU0_S = 4 * M_PI * 1e-7;   // mag/constants.go:8
 static constexpr int NREGION = 256;
 static constexpr int SYMLUT = NREGION * (NREGION + 1) / 2;
 
@@ -1099,7 +1098,7 @@ struct Sim : SimBase {
       a.nrm = sidx == 1 ? nullptr : tN(kk, sidx - 2);
       a.c5 = sidx == 2 ? T(1. / 6.) * h : T(1. / 3.) * h;
       a.cs = sidx == 4 ? T(1.) * h : T(1. / 2.) * h;
-      a.mu0 = (T)MU0_S;
+      a.mu0 = (T)MU0;
       a.gms = gms;
       a.gbext = part;
       a.N = n;
@@ -1107,7 +1106,7 @@ struct Sim : SimBase {
         // D = K * (Ms w) = K * gB: the forward plan with the mu0 Ms input scaling undone
         void *B[3] = {D, D + n, D + 2 * n};
         const void *mv[3] = {w, w + n, w + 2 * n};
-        demag_exec(demag, B, mv, nullptr, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul / MU0_S, st);
+        demag_exec(demag, B, mv, nullptr, p[UM_P_MSAT][0].arr.p, p[UM_P_MSAT][0].mul / MU0, st);
         for (int c = 0; c < 3; c++) a.D[c] = D + c * n;
       }
       launch_adj_stage(a, st);

@@ -400,7 +400,7 @@ struct BErrV {
           nan |= (e2 != e2);
           m0 = fmax(m0, e2);
           m1 = fmax(m1, k2);
-          } else if (MODE == 1) {
+        } else if (MODE == 1) {
           const double dx = (double)(x[0][0][w] - x[1][0][w]);
           const double dy = (double)(x[0][1][w] - x[1][1][w]);
           const double dz = (double)(x[0][2][w] - x[1][2][w]);
