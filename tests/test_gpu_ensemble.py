@@ -245,7 +245,7 @@ def test_batched_256_properties(gpu):
 
 
 def test_batched_short_runs_and_eager_members(gpu):
-    """n = 0, 1, 2 (no pair to replay after the eager step) and a member not in
+    """n = 0, 1, 2 (nothing, or two steps of two members, to step eagerly) and a member not in
     graph mode (stepped eagerly) next to batched ones: every member matches its
     twin stepped alone."""
     mix = [((32, 32, 2), "heun", np.float32), ((64, 32, 1), "rk45dp", np.float32)]
