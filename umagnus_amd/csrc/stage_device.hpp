@@ -33,8 +33,9 @@ __device__ __forceinline__ void stage_pair_n(const StageArgs<T> &s, int c, long 
 #pragma unroll
       for (int k = 0; k < NS; k++) u[k] = w ? x[e][k].y : x[e][k].x;
       T acc = f[0] * u[0];
-      if (NS == 3 && s.group3) {
-        acc = acc + fma(f[1], u[1], f[2] * u[2]);
+      if constexpr (NS == 3) {   // both orders: a branch for each component would wait for its loads
+        const T g = acc + fma(f[1], u[1], f[2] * u[2]), q = fma(f[2], u[2], fma(f[1], u[1], acc));
+        acc = s.group3 ? g : q;
       } else {
 #pragma unroll
         for (int k = 1; k < NS; k++) acc = fma(f[k], u[k], acc);
